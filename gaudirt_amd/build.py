@@ -27,8 +27,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # The host pass warns that it does not know the feature.
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 # Tuning variants of the kernels as extra -D flags, e.g.
-# GAUDIRT_AMD_DEFINES="-DGK_PREFILL_MFMA32=1" (the 32 x 32 prefill variant);
-# empty for the shipping build.
+# GAUDIRT_AMD_DEFINES="-DGK_STREAM_UNIT_COST=4" (the decode schedule's charge
+# per unit); empty for the shipping build.
 DEFINES = os.environ.get("GAUDIRT_AMD_DEFINES", "").split()
 COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-I", str(ROOT / "include"), "-I", str(CSRC),
           "-Wall", "-Wno-unused-function", *DEFINES]
