@@ -31,6 +31,7 @@ STREAM_UNIT_COST = 2
 EXPORTED = [
     "gk_last_error", "gk_version", "gk_kv_store", "gk_paged_decode_workspace_bytes",
     "gk_paged_decode_partition_tokens", "gk_paged_decode", "gk_paged_decode_scratch", "gk_paged_prefill",
+    "gk_prefill_list_build", "gk_prefill_list_workspace_bytes", "gk_paged_prefill_listed",
     "gk_split_k_merge",
     "gk_attn_tile_indices", "gk_advance_decode_lengths",
     "gk_metadata_workspace_bytes", "gk_metadata_normalize", "gk_block_tables",
@@ -81,6 +82,14 @@ class PrefillParams(_Sized):
         ("q_heads", c_i32), ("kv_heads", c_i32), ("head_dim", c_i32),
         ("scale", c_f32), ("softcap", c_f32), ("sliding_window", c_i32),
         ("out", c_void_p), ("out_row_stride", c_i64),
+    ]
+
+
+class PrefillList(_Sized):
+    _fields_ = [
+        ("struct_size", ctypes.c_size_t),
+        ("items", c_void_p), ("merges", c_void_p), ("row_request", c_void_p),
+        ("item_count", c_i32), ("merge_count", c_i32), ("part_slots", c_i32),
     ]
 
 
@@ -155,6 +164,11 @@ def load():
     lib.gk_paged_decode.argtypes = [ctypes.POINTER(DecodeParams), c_void_p, ctypes.c_size_t, c_void_p]
     lib.gk_paged_decode_scratch.argtypes = [ctypes.POINTER(DecodeParams), c_void_p]
     lib.gk_paged_prefill.argtypes = [ctypes.POINTER(PrefillParams), c_void_p]
+    lib.gk_prefill_list_build.argtypes = [c_void_p] * 3 + [c_i32] * 5 + [c_void_p, c_i64, ctypes.POINTER(PrefillList)]
+    lib.gk_prefill_list_workspace_bytes.restype = ctypes.c_size_t
+    lib.gk_prefill_list_workspace_bytes.argtypes = [ctypes.POINTER(PrefillParams), ctypes.POINTER(PrefillList)]
+    lib.gk_paged_prefill_listed.argtypes = [ctypes.POINTER(PrefillParams), ctypes.POINTER(PrefillList), c_void_p,
+                                            ctypes.c_size_t, c_void_p]
     lib.gk_kv_store.argtypes = [c_void_p, c_void_p, c_i64, c_i64, c_void_p, c_i32, c_void_p, c_i64, c_i32, c_i32,
                                 c_void_p]
     lib.gk_split_k_merge.argtypes = [c_void_p, c_void_p, c_void_p, c_i32, c_i32, c_i32, c_i32, c_void_p, c_i64,

@@ -7,7 +7,8 @@
 // every key is read through the block table.
 //
 // Work decomposition. A workgroup of eight waves owns one (sequence, kv head,
-// tile of rows). The GQA group is folded into the tile: its 256 "query rows"
+// tile of rows), or with a work list (prefill_schedule.hpp) a range of such a
+// tile's keys, whose partial result prefill_merge_kernel combines. The GQA group is folded into the tile: its 256 "query rows"
 // (128 at head_dim 256) are (row, head) pairs, so one K/V tile serves every
 // head of the group. Each wave computes 32 query rows (two 16-column MFMA
 // tiles; one, 16 rows, at head_dim 256) against the keys of a step (64 at
@@ -26,10 +27,14 @@
 // fp32 accumulation, one normalisation at the end by the sum of those bf16
 // probabilities, bf16 output.
 #include "gk_mfma.hpp"
+#include "prefill_schedule.hpp"
 #include "work_order.hpp"
 
 #include <algorithm>
+#include <cstring>
+#include <new>
 #include <type_traits>
+#include <vector>
 
 namespace gk {
 namespace {
@@ -52,15 +57,17 @@ constexpr int kNT = 2;
 constexpr int kQrowsPerWave = 16 * kNT;
 template <int D>
 constexpr int prefill_nt() { return D > 128 ? 1 : kNT; }
-// Query rows per workgroup at head dimension d.
-constexpr int prefill_qrows(int d) { return kPrefillWaves * 16 * (d > 128 ? 1 : kNT); }
+static_assert(prefill_tile_qrows(64) == kPrefillWaves * 16 * prefill_nt<64>() &&
+                  prefill_tile_qrows(128) == kPrefillWaves * 16 * prefill_nt<128>() &&
+                  prefill_tile_qrows(256) == kPrefillWaves * 16 * prefill_nt<256>(),
+              "the schedule's row tiles are the kernel's");
 // Keys per step: 64 at head_dim 128 (half the per-step barriers, cross-lane
 // maxima, re-base checks and load setup of 32-key steps: C4 178.1 -> 166.8
 // us); 32 at head_dim 64, whose 64-key form needs 130 VGPRs and so would drop
 // from four waves per SIMD to three, and at head_dim 256, where a 64-key K
 // and V tile pair takes 64 KiB of LDS per stage.
 template <int D>
-constexpr int prefill_keys() { return D == 128 ? 64 : 32; }
+constexpr int prefill_keys() { return prefill_step_keys(D); }
 // K/V pipeline depth. Two: three and four stages measured the same on C4 (the
 // kernel is bound by its instruction stream, not by load latency).
 constexpr int kStages = 2;
@@ -88,6 +95,18 @@ struct PrefillArgs {
   uint16_t* out;
   int64_t out_stride;
   DivMagic tiles_div, seqs_div, group_div;  // division by tiles, seqs and group (work_order.hpp)
+  // Work list (prefill_schedule.hpp) instead of the sequence arrays when not null.
+  const int32_t* items;
+  const int32_t* row_request;  // block-table row of each query row
+  int32_t item_count;
+  // XCD x serves the kv heads h with h % classes == x % classes, classes =
+  // gcd(kv_heads, 8): class_heads = kv_heads / classes heads on class_xcds =
+  // 8 / classes XCDs (class_shift = log2 classes).
+  int32_t class_shift, class_heads, class_xcds;
+  DivMagic class_heads_div;
+  int32_t part_slots;          // partial slots of one kv head
+  float* part_o;               // [kv head, slot][wave][query tile][16-dim chunk][lane] x 4 output rows
+  float* part_ml;              // [kv head, slot][wave][query tile][2][16]: base (log2 units), sum
 };
 
 template <int D>
@@ -154,34 +173,80 @@ __global__ __launch_bounds__(kPrefillWaves * 64, 1) void prefill_kernel(PrefillA
   // early-exit test (the compiler would otherwise fetch the sequence pointers
   // after the work-item arithmetic and the fields one by one: six round trips
   // before the first K/V load instead of three).
-  asm volatile("" ::"s"(a.seq_rows), "s"(a.seq_prefix), "s"(a.seq_first_row), "s"(a.seq_request),
-               "s"(a.block_tables), "s"(a.query), "s"(a.pool), "s"(a.out), "s"(a.tiles), "s"(a.seqs),
-               "s"(a.rows_per_tile), "s"(a.group), "s"(a.bt_stride), "s"(a.block_shift), "s"(a.window),
-               "s"(a.q_stride), "s"(a.slots), "s"(a.kv_heads), "s"(gridDim.x), "s"(a.tiles_div.mul),
-               "s"(a.tiles_div.shift), "s"(a.seqs_div.mul), "s"(a.seqs_div.shift), "s"(a.group_div.mul),
-               "s"(a.group_div.shift));
-  const int nitems = gridDim.x, xcd = blockIdx.x % kXcds, per_xcd = nitems / kXcds, extra = nitems % kXcds;
-  // Divisions by runtime values go through the host's multiply-shift pairs.
-  const auto div_tiles = [&](int x) { return (int)fast_div((uint32_t)x, a.tiles_div); };
-  const auto div_group = [&](int x) { return (int)fast_div((uint32_t)x, a.group_div); };
-  const int item = heavy_first_item(xcd * per_xcd + min(xcd, extra), per_xcd + (xcd < extra), a.tiles,
-                                    (int)blockIdx.x / kXcds, div_tiles);
-  const int item_seq = div_tiles(item), tile = item - item_seq * a.tiles;
-  const int kvh = (int)fast_div((uint32_t)item_seq, a.seqs_div), seq = item_seq - kvh * a.seqs;
-  const int rows = a.seq_rows[seq], prefix = a.seq_prefix[seq], seq_first = a.seq_first_row[seq];
-  const int request = a.seq_request[seq];
-  asm volatile("" ::"s"(rows), "s"(prefix), "s"(seq_first), "s"(request));
-  const int r0 = tile * a.rows_per_tile;
-  if (r0 >= rows) return;
-  const int nr = min(a.rows_per_tile, rows - r0);
-  const int first_row = seq_first + r0;
-  const int32_t* __restrict__ bt = a.block_tables + (int64_t)request * a.bt_stride;
+  // A work list's record holds all of that in one load.
   const int g = a.group;
-  const int pos_lo = prefix + r0, pos_hi = prefix + r0 + nr - 1;
-  const int key_end = pos_hi + 1;
-  const int key_begin = a.window > 0 ? max(0, pos_lo - a.window + 1) : 0;
-  const int kb0 = key_begin & ~(kKeys - 1);
-  const int nsteps = (key_end - kb0 + kKeys - 1) / kKeys;
+  const auto div_group = [&](int x) { return (int)fast_div((uint32_t)x, a.group_div); };
+  int kvh, request, first_row, nr, pos_lo, key_begin, kb0, nsteps, slot = -1;
+  if (a.items) {
+    asm volatile("" ::"s"(a.items), "s"(a.row_request), "s"(a.item_count), "s"(a.class_shift), "s"(a.class_heads),
+                 "s"(a.class_xcds), "s"(a.class_heads_div.mul), "s"(a.class_heads_div.shift), "s"(a.part_slots),
+                 "s"(a.block_tables), "s"(a.query), "s"(a.pool), "s"(a.out), "s"(a.group), "s"(a.bt_stride),
+                 "s"(a.block_shift), "s"(a.window), "s"(a.q_stride), "s"(a.slots), "s"(a.kv_heads),
+                 "s"(a.group_div.mul), "s"(a.group_div.shift));
+    // Item j of this XCD: the list is dealt out over the XCDs of the class,
+    // longest items first, the class's kv heads side by side.
+    const int xcd = blockIdx.x % kXcds, j = blockIdx.x / kXcds;
+    const int jl = (int)fast_div((uint32_t)j, a.class_heads_div);
+    const int li = jl * a.class_xcds + (xcd >> a.class_shift);
+    kvh = (xcd & ((1 << a.class_shift) - 1)) + ((j - jl * a.class_heads) << a.class_shift);
+    if (li >= a.item_count) return;
+    const int32_t* rec = a.items + (int64_t)li * kPrefillItemWords;
+    first_row = scalar_load(rec, 0);
+    nr = scalar_load(rec, 1);
+    pos_lo = scalar_load(rec, 2);
+    const int key0 = scalar_load(rec, 3);
+    nsteps = scalar_load(rec, 4);
+    slot = scalar_load(rec, 5);
+    request = scalar_load(a.row_request, first_row);
+    // The list may be made for a wider window than the call's: steps that lie
+    // before every row's window are skipped.
+    const int left = a.window > 0 ? max(0, pos_lo - a.window + 1) : 0;
+    kb0 = max(key0, left & ~(kKeys - 1));
+    nsteps -= (kb0 - key0) / kKeys;
+    key_begin = max(left, kb0);
+    if (nsteps <= 0) {
+      // No visible key in this piece (never a whole item): an empty partial,
+      // whose output the merge does not read into its sums.
+      if (slot >= 0 && lane < 16) {
+        float* ml = a.part_ml + (((int64_t)kvh * a.part_slots + slot) * kPrefillWaves + wave) * (kNT * 32);
+#pragma unroll
+        for (int nt = 0; nt < kNT; ++nt) {
+          ml[nt * 32 + lane] = -INFINITY;
+          ml[nt * 32 + 16 + lane] = 0.f;
+        }
+      }
+      return;
+    }
+  } else {
+    asm volatile("" ::"s"(a.seq_rows), "s"(a.seq_prefix), "s"(a.seq_first_row), "s"(a.seq_request),
+                 "s"(a.block_tables), "s"(a.query), "s"(a.pool), "s"(a.out), "s"(a.tiles), "s"(a.seqs),
+                 "s"(a.rows_per_tile), "s"(a.group), "s"(a.bt_stride), "s"(a.block_shift), "s"(a.window),
+                 "s"(a.q_stride), "s"(a.slots), "s"(a.kv_heads), "s"(gridDim.x), "s"(a.tiles_div.mul),
+                 "s"(a.tiles_div.shift), "s"(a.seqs_div.mul), "s"(a.seqs_div.shift), "s"(a.group_div.mul),
+                 "s"(a.group_div.shift));
+    const int nitems = gridDim.x, xcd = blockIdx.x % kXcds, per_xcd = nitems / kXcds, extra = nitems % kXcds;
+    // Divisions by runtime values go through the host's multiply-shift pairs.
+    const auto div_tiles = [&](int x) { return (int)fast_div((uint32_t)x, a.tiles_div); };
+    const int item = heavy_first_item(xcd * per_xcd + min(xcd, extra), per_xcd + (xcd < extra), a.tiles,
+                                      (int)blockIdx.x / kXcds, div_tiles);
+    const int item_seq = div_tiles(item), tile = item - item_seq * a.tiles;
+    kvh = (int)fast_div((uint32_t)item_seq, a.seqs_div);
+    const int seq = item_seq - kvh * a.seqs;
+    const int rows = a.seq_rows[seq], prefix = a.seq_prefix[seq], seq_first = a.seq_first_row[seq];
+    request = a.seq_request[seq];
+    asm volatile("" ::"s"(rows), "s"(prefix), "s"(seq_first), "s"(request));
+    const int r0 = tile * a.rows_per_tile;
+    if (r0 >= rows) return;
+    nr = min(a.rows_per_tile, rows - r0);
+    first_row = seq_first + r0;
+    pos_lo = prefix + r0;
+    key_begin = a.window > 0 ? max(0, pos_lo - a.window + 1) : 0;
+    kb0 = key_begin & ~(kKeys - 1);
+    nsteps = (pos_lo + nr - kb0 + kKeys - 1) / kKeys;
+  }
+  const int32_t* __restrict__ bt = a.block_tables + (int64_t)request * a.bt_stride;
+  // Keys of this workgroup: [key_begin, key_end), a whole item's or a piece's.
+  const int key_end = min(pos_lo + nr, kb0 + nsteps * kKeys);
 
   // This lane's query rows (one per 16-column tile): qrow = (row, head).
   int qpos[kNT], qleft[kNT];
@@ -594,6 +659,28 @@ __global__ __launch_bounds__(kPrefillWaves * 64, 1) void prefill_kernel(PrefillA
     if (lead) __syncthreads();
   }
 
+  if (slot >= 0) {
+    // A piece: its accumulators, bases and sums as they stand in registers
+    // (1 KiB stores; the merge kernel reads them back in the same layout).
+    const int64_t pslot = (int64_t)kvh * a.part_slots + slot;
+#pragma unroll
+    for (int nt = 0; nt < kNT; ++nt) {
+      const int t = wave * kNT + nt;  // 16-row tile of the workgroup
+      if (div_group(16 * t) >= nr) break;
+      f32x4_t* po = reinterpret_cast<f32x4_t*>(a.part_o) + ((pslot * (kPrefillWaves * kNT) + t) * S::NO) * 64 + lane;
+#pragma unroll
+      for (int c = 0; c < S::NO; ++c) po[c * 64] = o[nt][c];
+      float* ml = a.part_ml + (pslot * (kPrefillWaves * kNT) + t) * 32;
+      if (lane < 16) ml[lane] = m_run[nt];
+      if constexpr (kMfmaSum) {
+        if (c16 == 0) *reinterpret_cast<f32x4_t*>(ml + 16 + 4 * q) = l_run[nt];
+      } else {
+        const float l = col4_sum(l_run[nt][0]);
+        if (lane < 16) ml[16 + lane] = l;
+      }
+    }
+    return;
+  }
   // Normalise into bf16 rows in LDS: o row 4q + r of tile nt, its sum in
   // l_run[nt][r] (MFMA sums) or in lane c16 == 4q + r after the cross-row sum
   // (VALU sums). Then each wave stores its own rows as 16-byte pieces: the
@@ -632,6 +719,93 @@ __global__ __launch_bounds__(kPrefillWaves * 64, 1) void prefill_kernel(PrefillA
   }
 }
 
+// ---------------------------------------------------------------------------
+// Merge of the items that a work list splits
+// ---------------------------------------------------------------------------
+struct PrefillMergeArgs {
+  const int32_t* merges;  // PrefillMerge records
+  int32_t part_slots, group, q_heads;
+  DivMagic group_div;
+  const float* part_o;
+  const float* part_ml;
+  uint16_t* out;
+  int64_t out_stride;
+};
+
+// Bound by reading the partials (from the last-level cache mostly) and, for few
+// of them, by the launch: 8 us for 256 partials of 128 KiB (4.2 TB/s), 15 us for
+// 496 (4.4 TB/s), 7 us for 258 of 64 KiB. One wave per (split item, kv head, 16 query rows, 32
+// dims): the partials are read as the pieces' lanes stored them, 1 KiB a load,
+// the loads of up to eight parts in one memory round trip.
+template <int D>
+__global__ __launch_bounds__(64) void prefill_merge_kernel(PrefillMergeArgs a) {
+  constexpr int kTiles = prefill_tile_qrows(D) / 16, NO = D / 16, CC = 2, kGroups = NO / CC;
+  constexpr int kRowBytes = 16 * CC * 2 + 16;
+  __shared__ __attribute__((aligned(16))) char lds[16 * kRowBytes];
+  const int lane = threadIdx.x, q = lane >> 4, c16 = lane & 15;
+  const int mi = blockIdx.x / (kTiles * kGroups), rest = blockIdx.x % (kTiles * kGroups);
+  const int t = rest / kGroups, cg = rest % kGroups, kvh = blockIdx.y;
+  const int32_t* rec = a.merges + (int64_t)mi * kPrefillMergeWords;
+  const int first_row = scalar_load(rec, 0), nr = scalar_load(rec, 1), slot = scalar_load(rec, 2),
+            parts = scalar_load(rec, 3);
+  if ((int)fast_div((uint32_t)(16 * t), a.group_div) >= nr) return;
+  const int64_t tile0 = ((int64_t)kvh * a.part_slots + slot) * kTiles + t;  // part p: + p kTiles
+  f32x4_t m_run, l_run{0.f, 0.f, 0.f, 0.f}, acc[CC];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) m_run[r] = -INFINITY;
+#pragma unroll
+  for (int c = 0; c < CC; ++c) acc[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  auto merge_parts = [&](auto batch) {
+    constexpr int BATCH = decltype(batch)::value;
+    for (int p0 = 0; p0 < parts; p0 += BATCH) {
+      f32x4_t mp[BATCH], lp[BATCH], op[BATCH][CC];
+#pragma unroll
+      for (int u = 0; u < BATCH; ++u) {
+        const int64_t tile = tile0 + (int64_t)min(p0 + u, parts - 1) * kTiles;
+        mp[u] = *reinterpret_cast<const f32x4_t*>(a.part_ml + tile * 32 + 4 * q);
+        lp[u] = *reinterpret_cast<const f32x4_t*>(a.part_ml + tile * 32 + 16 + 4 * q);
+        const f32x4_t* po = reinterpret_cast<const f32x4_t*>(a.part_o) + (tile * NO + cg * CC) * 64 + lane;
+#pragma unroll
+        for (int c = 0; c < CC; ++c) op[u][c] = po[c * 64];
+      }
+#pragma unroll
+      for (int u = 0; u < BATCH; ++u) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          // Parts past the last (clamped duplicates) weigh nothing. A part
+          // without a visible key has no output: its slot is not read into
+          // the sum.
+          const float mu = p0 + u < parts ? mp[u][r] : -INFINITY;
+          const float mn = fmaxf(m_run[r], mu);
+          const float fa = m_run[r] == -INFINITY ? 0.f : fast_exp2(m_run[r] - mn);
+          const float fb = mu == -INFINITY ? 0.f : fast_exp2(mu - mn);
+          l_run[r] = l_run[r] * fa + (mu == -INFINITY ? 0.f : lp[u][r] * fb);
+#pragma unroll
+          for (int c = 0; c < CC; ++c) acc[c][r] = acc[c][r] * fa + (mu == -INFINITY ? 0.f : op[u][c][r] * fb);
+          m_run[r] = mn;
+        }
+      }
+    }
+  };
+  if (parts <= 4) merge_parts(std::integral_constant<int, 4>{});
+  else merge_parts(std::integral_constant<int, 8>{});
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float inv = l_run[r] > 0.f ? 1.f / l_run[r] : 0.f;
+    __bf16* dst = reinterpret_cast<__bf16*>(lds + (4 * q + r) * kRowBytes) + c16;
+#pragma unroll
+    for (int c = 0; c < CC; ++c) dst[16 * c] = (__bf16)(acc[c][r] * inv);
+  }
+  // The wave's own LDS operations complete in order: 16 rows x 4 pieces of 16 bytes.
+  static_assert(CC == 2, "one 16-byte piece per lane");
+  const int ql = lane >> 2, part = lane & 3;
+  const uint4 v = *reinterpret_cast<const uint4*>(lds + ql * kRowBytes + part * 16);
+  const int qr = 16 * t + ql, row = (int)fast_div((uint32_t)qr, a.group_div), head = qr - row * a.group;
+  if (row < nr)
+    *reinterpret_cast<uint4*>(a.out + (int64_t)(first_row + row) * a.out_stride +
+                              (int64_t)(kvh * a.group + head) * D + cg * (16 * CC) + part * 8) = v;
+}
+
 template <int D, int MODE>
 void launch_mode(const PrefillArgs& a, bool softcap, dim3 grid, hipStream_t stream) {
   if (softcap) prefill_kernel<D, true, MODE><<<grid, kPrefillWaves * 64, 0, stream>>>(a);
@@ -648,7 +822,9 @@ void launch(const PrefillArgs& a, bool softcap, int block_size, dim3 grid, hipSt
 
 }  // namespace
 
-int paged_prefill(const gk_prefill_params* p, hipStream_t stream) {
+namespace {
+
+int validate(const gk_prefill_params* p, bool listed) {
   if (!p) return fail(GK_ERR_INVALID_ARGUMENT, "gk_paged_prefill: null parameters");
   if (p->struct_size != sizeof(gk_prefill_params))
     return fail(GK_ERR_INVALID_ARGUMENT, "gk_paged_prefill: struct_size does not match this library's gk_prefill_params");
@@ -664,15 +840,20 @@ int paged_prefill(const gk_prefill_params* p, hipStream_t stream) {
     return fail(GK_ERR_UNSUPPORTED, "gk_paged_prefill: one kv head's K or V region must stay below 4 GiB");
   if (!(p->scale > 0.f) || !(p->scale < INFINITY) || !(p->softcap >= 0.f) || !(p->softcap < INFINITY))
     return fail(GK_ERR_INVALID_ARGUMENT, "gk_paged_prefill: invalid scale or softcap");
-  if (p->seqs == 0 || p->max_rows == 0) return GK_OK;
-  if (!p->query || !p->pool || !p->block_tables || !p->seq_request || !p->seq_first_row || !p->seq_rows ||
-      !p->seq_prefix || !p->out)
+  if (!listed && (p->seqs == 0 || p->max_rows == 0)) return GK_OK;
+  if (!p->query || !p->pool || !p->block_tables || !p->out ||
+      (!listed && (!p->seq_request || !p->seq_first_row || !p->seq_rows || !p->seq_prefix)))
     return fail(GK_ERR_INVALID_ARGUMENT, "gk_paged_prefill: null pointer");
   const auto misaligned = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) != 0; };
   if (misaligned(p->query) || misaligned(p->pool) || misaligned(p->out) || (p->q_row_stride & 7) ||
       (p->out_row_stride & 7) || p->q_row_stride < (int64_t)p->q_heads * p->head_dim ||
       p->out_row_stride < (int64_t)p->q_heads * p->head_dim)
     return fail(GK_ERR_INVALID_ARGUMENT, "gk_paged_prefill: query/pool/out must be 16-byte aligned with full rows");
+  return GK_OK;
+}
+
+// The arguments that do not depend on where the work comes from.
+PrefillArgs common_args(const gk_prefill_params* p) {
   PrefillArgs a{};
   a.query = static_cast<const uint16_t*>(p->query);
   a.q_stride = p->q_row_stride;
@@ -681,32 +862,148 @@ int paged_prefill(const gk_prefill_params* p, hipStream_t stream) {
   a.block_tables = p->block_tables;
   a.bt_stride = p->bt_stride;
   a.block_shift = log2_int(p->block_size);
-  a.seq_request = p->seq_request;
-  a.seq_first_row = p->seq_first_row;
-  a.seq_rows = p->seq_rows;
-  a.seq_prefix = p->seq_prefix;
   a.q_heads = p->q_heads;
   a.kv_heads = p->kv_heads;
   a.group = p->q_heads / p->kv_heads;
-  a.rows_per_tile = prefill_qrows(p->head_dim) / a.group;
-  a.tiles = (p->max_rows + a.rows_per_tile - 1) / a.rows_per_tile;
-  a.seqs = p->seqs;
+  a.rows_per_tile = prefill_tile_qrows(p->head_dim) / a.group;
   const bool softcap = p->softcap > 0.f;
   a.score_scale = softcap ? p->scale / p->softcap : p->scale * kLog2e;
   a.softcap_log2 = p->softcap * kLog2e;
   a.window = p->sliding_window > 0 ? p->sliding_window : 0;
   a.out = static_cast<uint16_t*>(p->out);
   a.out_stride = p->out_row_stride;
-  a.tiles_div = div_magic((uint32_t)a.tiles);
-  a.seqs_div = div_magic((uint32_t)a.seqs);
   a.group_div = div_magic((uint32_t)a.group);
-  const int64_t items = (int64_t)a.tiles * p->kv_heads * p->seqs;
-  if (items > (int64_t)1 << 30) return fail(GK_ERR_INVALID_ARGUMENT, "gk_paged_prefill: too many rows");
-  const dim3 grid((unsigned)items);
+  return a;
+}
+
+int launch_prefill(const gk_prefill_params* p, const PrefillArgs& a, int64_t workgroups, hipStream_t stream) {
+  const dim3 grid((unsigned)workgroups);
+  const bool softcap = p->softcap > 0.f;
   if (p->head_dim == 64) launch<64>(a, softcap, p->block_size, grid, stream);
   else if (p->head_dim == 128) launch<128>(a, softcap, p->block_size, grid, stream);
   else launch<256>(a, softcap, p->block_size, grid, stream);
   return hip_status(hipGetLastError(), "gk_paged_prefill launch");
+}
+
+// Workspace of a work list: the partial outputs, then (base, sum) of every row.
+size_t list_output_bytes(const gk_prefill_params* p, const gk_prefill_list* list) {
+  return (size_t)p->kv_heads * list->part_slots * prefill_tile_qrows(p->head_dim) * p->head_dim * sizeof(float);
+}
+size_t list_workspace_bytes(const gk_prefill_params* p, const gk_prefill_list* list) {
+  return list_output_bytes(p, list) +
+         (size_t)p->kv_heads * list->part_slots * prefill_tile_qrows(p->head_dim) * 2 * sizeof(float);
+}
+
+}  // namespace
+
+int device_cus();
+
+int paged_prefill(const gk_prefill_params* p, hipStream_t stream) {
+  if (int rc = validate(p, false)) return rc;
+  if (p->seqs == 0 || p->max_rows == 0) return GK_OK;
+  PrefillArgs a = common_args(p);
+  a.seq_request = p->seq_request;
+  a.seq_first_row = p->seq_first_row;
+  a.seq_rows = p->seq_rows;
+  a.seq_prefix = p->seq_prefix;
+  a.seqs = p->seqs;
+  a.tiles = (p->max_rows + a.rows_per_tile - 1) / a.rows_per_tile;
+  a.tiles_div = div_magic((uint32_t)a.tiles);
+  a.seqs_div = div_magic((uint32_t)a.seqs);
+  const int64_t items = (int64_t)a.tiles * p->kv_heads * p->seqs;
+  if (items > (int64_t)1 << 30) return fail(GK_ERR_INVALID_ARGUMENT, "gk_paged_prefill: too many rows");
+  return launch_prefill(p, a, items, stream);
+}
+
+int paged_prefill_listed(const gk_prefill_params* p, const gk_prefill_list* list, void* workspace,
+                         size_t workspace_bytes, hipStream_t stream) {
+  if (int rc = validate(p, true)) return rc;
+  if (!list || list->struct_size != sizeof(gk_prefill_list))
+    return fail(GK_ERR_INVALID_ARGUMENT, "gk_paged_prefill_listed: struct_size does not match this library's gk_prefill_list");
+  if (list->item_count < 0 || list->merge_count < 0 || list->part_slots < 0 || list->part_slots > (1 << 20) ||
+      list->merge_count > (1 << 20))
+    return fail(GK_ERR_INVALID_ARGUMENT, "gk_paged_prefill_listed: list counts out of range");
+  if (list->item_count == 0) return GK_OK;
+  if (!list->items || !list->row_request || (list->merge_count && !list->merges))
+    return fail(GK_ERR_INVALID_ARGUMENT, "gk_paged_prefill_listed: null pointer");
+  if (list->part_slots && (!workspace || workspace_bytes < list_workspace_bytes(p, list) ||
+                           (reinterpret_cast<uintptr_t>(workspace) & 15)))
+    return fail(GK_ERR_WORKSPACE, "gk_paged_prefill_listed: workspace too small or not 16-byte aligned (" +
+                                      std::to_string(list_workspace_bytes(p, list)) + " bytes needed)");
+  PrefillArgs a = common_args(p);
+  a.items = list->items;
+  a.item_count = list->item_count;
+  a.row_request = list->row_request;
+  int classes = kXcds;
+  while (p->kv_heads % classes) classes /= 2;
+  a.class_shift = log2_int(classes);
+  a.class_heads = p->kv_heads / classes;
+  a.class_xcds = kXcds / classes;
+  a.class_heads_div = div_magic((uint32_t)a.class_heads);
+  a.part_slots = list->part_slots;
+  a.part_o = static_cast<float*>(workspace);
+  a.part_ml = reinterpret_cast<float*>(static_cast<char*>(workspace) + list_output_bytes(p, list));
+  const int64_t per_xcd = ((int64_t)list->item_count + a.class_xcds - 1) / a.class_xcds * a.class_heads;
+  if (per_xcd * kXcds > (int64_t)1 << 30)
+    return fail(GK_ERR_INVALID_ARGUMENT, "gk_paged_prefill_listed: too many items");
+  if (int rc = launch_prefill(p, a, per_xcd * kXcds, stream)) return rc;
+  if (!list->merge_count) return GK_OK;
+  PrefillMergeArgs m{};
+  m.merges = list->merges;
+  m.part_slots = list->part_slots;
+  m.group = a.group;
+  m.q_heads = p->q_heads;
+  m.group_div = a.group_div;
+  m.part_o = a.part_o;
+  m.part_ml = a.part_ml;
+  m.out = a.out;
+  m.out_stride = a.out_stride;
+  const int waves = prefill_tile_qrows(p->head_dim) / 16 * (p->head_dim / 32);
+  const dim3 grid((unsigned)(list->merge_count * waves), (unsigned)p->kv_heads);
+  if (p->head_dim == 64) prefill_merge_kernel<64><<<grid, 64, 0, stream>>>(m);
+  else if (p->head_dim == 128) prefill_merge_kernel<128><<<grid, 64, 0, stream>>>(m);
+  else prefill_merge_kernel<256><<<grid, 64, 0, stream>>>(m);
+  return hip_status(hipGetLastError(), "gk_paged_prefill_listed merge launch");
+}
+
+int prefill_list_build(const int32_t* seq_first_row, const int32_t* seq_rows, const int32_t* seq_prefix, int32_t seqs,
+                       int32_t q_heads, int32_t kv_heads, int32_t head_dim,
+                       int32_t sliding_window, int32_t* words, int64_t capacity, gk_prefill_list* list) {
+  if (!list || list->struct_size != sizeof(gk_prefill_list))
+    return fail(GK_ERR_INVALID_ARGUMENT, "gk_prefill_list_build: struct_size does not match this library's gk_prefill_list");
+  if ((head_dim != 64 && head_dim != 128 && head_dim != 256) || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads ||
+      q_heads / kv_heads > 128)
+    return fail(GK_ERR_INVALID_ARGUMENT, "gk_prefill_list_build: invalid head geometry");
+  if (seqs < 0 || seqs > 65535 || capacity < 0 || (seqs && (!seq_first_row || !seq_rows || !seq_prefix)))
+    return fail(GK_ERR_INVALID_ARGUMENT, "gk_prefill_list_build: invalid sequences");
+  int64_t rows = 0;
+  for (int32_t s = 0; s < seqs; ++s) {
+    if (seq_rows[s] < 0 || seq_prefix[s] < 0 || seq_first_row[s] < 0 ||
+        (int64_t)seq_prefix[s] + seq_rows[s] > INT32_MAX - 64)
+      return fail(GK_ERR_INVALID_ARGUMENT, "gk_prefill_list_build: invalid sequences");
+    rows += seq_rows[s];
+  }
+  if (rows > (1 << 20)) return fail(GK_ERR_INVALID_ARGUMENT, "gk_prefill_list_build: too many rows");
+  try {
+    std::vector<PrefillSeq> in(seqs);
+    for (int32_t s = 0; s < seqs; ++s)
+      in[s] = {seq_first_row[s], seq_rows[s], seq_prefix[s]};
+    const PrefillWorkList work = prefill_work_list(in.data(), seqs, q_heads / kv_heads, kv_heads, head_dim,
+                                                   sliding_window, device_cus());
+    list->item_count = (int32_t)work.items.size();
+    list->merge_count = (int32_t)work.merges.size();
+    list->part_slots = work.slots;
+    const int64_t item_words = (int64_t)work.items.size() * kPrefillItemWords,
+                  merge_words = (int64_t)work.merges.size() * kPrefillMergeWords;
+    if (!words || capacity < item_words + merge_words)
+      return fail(GK_ERR_WORKSPACE, "gk_prefill_list_build: the list needs " + std::to_string(item_words + merge_words) +
+                                        " words");
+    if (item_words) std::memcpy(words, work.items.data(), item_words * sizeof(int32_t));
+    if (merge_words) std::memcpy(words + item_words, work.merges.data(), merge_words * sizeof(int32_t));
+    return GK_OK;
+  } catch (const std::bad_alloc&) {
+    return fail(GK_ERR_OUT_OF_MEMORY, "gk_prefill_list_build: out of host memory");
+  }
 }
 
 }  // namespace gk
@@ -714,4 +1011,25 @@ int paged_prefill(const gk_prefill_params* p, hipStream_t stream) {
 extern "C" int gk_paged_prefill(const gk_prefill_params* params, hipStream_t stream) {
   gk::clear_error();
   return gk::paged_prefill(params, stream);
+}
+
+extern "C" int gk_prefill_list_build(const int32_t* seq_first_row, const int32_t* seq_rows, const int32_t* seq_prefix,
+                                     int32_t seqs, int32_t q_heads, int32_t kv_heads, int32_t head_dim,
+                                     int32_t sliding_window, int32_t* words, int64_t capacity, gk_prefill_list* list) {
+  gk::clear_error();
+  return gk::prefill_list_build(seq_first_row, seq_rows, seq_prefix, seqs, q_heads, kv_heads, head_dim, sliding_window,
+                                words, capacity, list);
+}
+
+extern "C" size_t gk_prefill_list_workspace_bytes(const gk_prefill_params* params, const gk_prefill_list* list) {
+  return params && list && params->struct_size == sizeof(gk_prefill_params) &&
+                 list->struct_size == sizeof(gk_prefill_list) && params->kv_heads > 0 && list->part_slots > 0
+             ? gk::list_workspace_bytes(params, list)
+             : 0;
+}
+
+extern "C" int gk_paged_prefill_listed(const gk_prefill_params* params, const gk_prefill_list* list, void* workspace,
+                                       size_t workspace_bytes, hipStream_t stream) {
+  gk::clear_error();
+  return gk::paged_prefill_listed(params, list, workspace, workspace_bytes, stream);
 }

@@ -230,9 +230,12 @@ struct PlanInfo {
   // batch row of each.
   int64_t decode_rows = 0, decode_max_context = 0;
   int64_t row_request_offset = 0, row_context_offset = 0, row_map_offset = 0;
-  // Runs of consecutive positions attended as MFMA tiles (gk_paged_prefill).
-  int64_t prefill_seqs = 0, prefill_max_rows = 0;
-  int64_t seq_request_offset = 0, seq_first_row_offset = 0, seq_rows_offset = 0, seq_prefix_offset = 0;
+  // Runs of consecutive positions attended as MFMA tiles: the work list of
+  // gk_paged_prefill_listed, whose items read their request from the
+  // metadata's own row requests.
+  int64_t prefill_items = 0, prefill_merges = 0, prefill_part_slots = 0;
+  int64_t prefill_items_offset = 0, prefill_merges_offset = 0;
+  at::Tensor prefill_row_request;
 };
 
 // Runs of at least this many consecutive positions go to the prefill kernel.
@@ -750,14 +753,12 @@ class PagedMetadata : public torch::CustomClassHolder {
     // device-built metadata are filled in on the device below.
     // The prefill kernel takes any page size, the token-granular map included.
     const bool prefill_ok = query_heads / kv_heads <= 128;
-    std::vector<int32_t> dec_request, dec_context, dec_map, seq_request, seq_first, seq_rows, seq_prefix;
+    std::vector<int32_t> dec_request, dec_context, dec_map, seq_first, seq_rows, seq_prefix, work;
     for (const auto& run : sequences_) {
       if (prefill_ok && run.length >= kPrefillMinRows) {
-        seq_request.push_back(host_map ? requests_h_[run.row] : 0);
         seq_first.push_back(run.row);
         seq_rows.push_back(run.length);
         seq_prefix.push_back(run.prefix);
-        info->prefill_max_rows = std::max<int64_t>(info->prefill_max_rows, run.length);
         continue;
       }
       for (int32_t i = run.row; i < run.row + run.length; ++i) {
@@ -789,11 +790,31 @@ class PagedMetadata : public torch::CustomClassHolder {
     info->row_request_offset = append(dec_request);
     info->row_context_offset = append(dec_context);
     info->row_map_offset = append(dec_map);
-    info->prefill_seqs = static_cast<int64_t>(seq_rows.size());
-    info->seq_request_offset = append(seq_request);
-    info->seq_first_row_offset = append(seq_first);
-    info->seq_rows_offset = append(seq_rows);
-    info->seq_prefix_offset = append(seq_prefix);
+    if (!seq_rows.empty()) {
+      gk_prefill_list list{};
+      list.struct_size = sizeof(list);
+      const auto build = [&] {
+        return gk_prefill_list_build(seq_first.data(), seq_rows.data(), seq_prefix.data(),
+                                     static_cast<int32_t>(seq_rows.size()),
+                                     static_cast<int32_t>(query_heads), static_cast<int32_t>(kv_heads),
+                                     static_cast<int32_t>(head_dim), static_cast<int32_t>(window), work.data(),
+                                     static_cast<int64_t>(work.size()), &list);
+      };
+      work.resize(4096);
+      int rc = build();
+      if (rc == GK_ERR_WORKSPACE) {
+        work.resize(int64_t{8} * list.item_count + int64_t{4} * list.merge_count);
+        rc = build();
+      }
+      check_gk(rc, "GaudiRT attention: prefill work list");
+      work.resize(int64_t{8} * list.item_count + int64_t{4} * list.merge_count);
+      info->prefill_items = list.item_count;
+      info->prefill_merges = list.merge_count;
+      info->prefill_part_slots = list.part_slots;
+      info->prefill_items_offset = append(work);
+      info->prefill_merges_offset = info->prefill_items_offset + int64_t{8} * list.item_count;
+      info->prefill_row_request = requests_;
+    }
     // Page 1: the request map itself is the block table, read in place.
     std::vector<int32_t> tables;
     if (page == 1) {
@@ -819,9 +840,6 @@ class PagedMetadata : public torch::CustomClassHolder {
       if (info->decode_rows && !all_decode)
         section(info->row_request_offset, info->decode_rows)
             .copy_(requests_.index_select(0, section(info->row_map_offset, info->decode_rows)));
-      if (info->prefill_seqs)
-        section(info->seq_request_offset, info->prefill_seqs)
-            .copy_(requests_.index_select(0, section(info->seq_first_row_offset, info->prefill_seqs)));
       if (page != 1)
         check_gk(gk_block_tables(mapping_.data_ptr<int32_t>(), static_cast<int32_t>(request_count_),
                                  static_cast<int32_t>(context_), static_cast<int32_t>(page),
@@ -977,7 +995,7 @@ at::Tensor paged_attn_impl(const at::Tensor& query, const at::Tensor& key, const
   }
   const int32_t* words = plan.storage.data_ptr<int32_t>();
   const int32_t sw = sliding_window > 0 ? static_cast<int32_t>(sliding_window) : -1;
-  if (plan.prefill_seqs) {
+  if (plan.prefill_items) {
     gk_prefill_params f{};
     f.struct_size = sizeof(f);
     f.query = q.data_ptr();
@@ -987,12 +1005,6 @@ at::Tensor paged_attn_impl(const at::Tensor& query, const at::Tensor& key, const
     f.block_tables = plan.block_tables(words);
     f.bt_stride = plan.bt_stride;
     f.block_size = static_cast<int32_t>(plan.block_size);
-    f.seq_request = words + plan.seq_request_offset;
-    f.seq_first_row = words + plan.seq_first_row_offset;
-    f.seq_rows = words + plan.seq_rows_offset;
-    f.seq_prefix = words + plan.seq_prefix_offset;
-    f.seqs = static_cast<int32_t>(plan.prefill_seqs);
-    f.max_rows = static_cast<int32_t>(plan.prefill_max_rows);
     f.q_heads = static_cast<int32_t>(plan.query_heads);
     f.kv_heads = static_cast<int32_t>(plan.kv_heads);
     f.head_dim = static_cast<int32_t>(head_dim);
@@ -1001,7 +1013,19 @@ at::Tensor paged_attn_impl(const at::Tensor& query, const at::Tensor& key, const
     f.sliding_window = sw;
     f.out = output.data_ptr();
     f.out_row_stride = output.stride(0);
-    check_gk(gk_paged_prefill(&f, stream), "GaudiRT attention (prefill)");
+    gk_prefill_list list{};
+    list.struct_size = sizeof(list);
+    list.items = words + plan.prefill_items_offset;
+    list.merges = words + plan.prefill_merges_offset;
+    list.row_request = plan.prefill_row_request.data_ptr<int32_t>();
+    list.item_count = static_cast<int32_t>(plan.prefill_items);
+    list.merge_count = static_cast<int32_t>(plan.prefill_merges);
+    list.part_slots = static_cast<int32_t>(plan.prefill_part_slots);
+    const size_t need = gk_prefill_list_workspace_bytes(&f, &list);
+    at::Tensor workspace;
+    if (need) workspace = at::empty({static_cast<int64_t>(need)}, query.options().dtype(at::kByte));
+    check_gk(gk_paged_prefill_listed(&f, &list, need ? workspace.data_ptr() : nullptr, need, stream),
+             "GaudiRT attention (prefill)");
   }
   if (plan.decode_rows) {
     gk_decode_params p{};

@@ -174,6 +174,37 @@ typedef struct gk_prefill_params {
 
 int gk_paged_prefill(const gk_prefill_params* params, hipStream_t stream);
 
+/* The same attention over a work list, for callers that know the sequence
+ * lengths on the host: items (row tile, key range) of about equal length fill
+ * the GPU also when the chunk has few rows or the last round of workgroups
+ * would be partly empty; an item cut along its keys leaves fp32 partials in the
+ * workspace, which a second launch merges (log-sum-exp). Replaces the reference's
+ * host-side work plan (src/bridge/attention_plan.cpp:199-237,262-335).
+ *
+ * gk_prefill_list_build (host only) writes the list for these sequences (host
+ * arrays, as gk_prefill_params' device arrays) and window into words:
+ * item_count records of 8 words, then merge_count records of 4. It sets the
+ * counts of `list` also when capacity is too small (GK_ERR_WORKSPACE). The
+ * caller copies the words to the device and sets items and merges to the two
+ * sections, and row_request to the block-table row of every query row (device).
+ * gk_paged_prefill_listed does not read seq_*, seqs and max_rows of its
+ * gk_prefill_params; its sliding_window is at least as narrow as the list's. */
+typedef struct gk_prefill_list {
+  size_t struct_size;          /* sizeof(gk_prefill_list) as the caller was built; checked */
+  const int32_t* items;
+  const int32_t* merges;
+  const int32_t* row_request;
+  int32_t item_count, merge_count;
+  int32_t part_slots;          /* partial slots per kv head */
+} gk_prefill_list;
+
+int gk_prefill_list_build(const int32_t* seq_first_row, const int32_t* seq_rows, const int32_t* seq_prefix,
+                          int32_t seqs, int32_t q_heads, int32_t kv_heads, int32_t head_dim, int32_t sliding_window,
+                          int32_t* words, int64_t capacity, gk_prefill_list* list);
+size_t gk_prefill_list_workspace_bytes(const gk_prefill_params* params, const gk_prefill_list* list);
+int gk_paged_prefill_listed(const gk_prefill_params* params, const gk_prefill_list* list, void* workspace,
+                            size_t workspace_bytes, hipStream_t stream);
+
 /* ---------------------------------------------------------------------------
  * Split-K merge on its own: combines `parts` fp32 partial states per (row, head)
  * into bf16 output. partial_out [rows, heads, max_parts, head_dim] holds
