@@ -37,6 +37,7 @@ struct DecodeArgs {
   int64_t out_stride;
   float* part_o;
   float* part_ml;
+  uint16_t* pool_out;  // the pool as a store target (decode_unit.hip)
 };
 
 template <int D>
@@ -49,6 +50,32 @@ struct MfmaShape {
   static constexpr int NO = D / 16;               // 16-dim output chunks of P.V
   static constexpr int TILE = TS * D * 2;         // bytes of one K or V tile in LDS
 };
+
+// A row's tiles: visible keys [left, ctx) occupy tiles first .. first + count - 1.
+// An empty row still owns one (fully masked) tile, so every unit is finalised.
+struct RowTiles {
+  int first, count, left, ctx;
+};
+
+template <int TS>
+__device__ __forceinline__ RowTiles row_tiles(int ctx, int window) {
+  RowTiles r;
+  r.ctx = ctx > 0 ? ctx : 0;
+  r.left = visible_left(r.ctx, window);
+  r.first = r.left / TS;
+  r.count = stream_row_tile_count(r.ctx, window, TS);
+  return r;
+}
+
+// One workgroup per unit (decode_unit.hip): rows of at most this many visible
+// keys (1 MiB of keys and values; at head_dim 64 what lets two workgroups share
+// a CU's LDS), whose block-table entries, one more when a window starts inside
+// a page, lie in LDS; and as many new rows with a fused store.
+constexpr int unit_max_keys(int head_dim) { return head_dim == 64 ? 3072 : (1 << 18) / head_dim; }
+constexpr int kUnitMaxNewRows = 256;
+bool unit_decode_fits(const gk_decode_params* params, int64_t units);
+int launch_unit_decode(const DecodeArgs& a, bool softcap, int head_dim, const gk_decode_params* params, bool store,
+                       hipStream_t stream);
 
 // Balanced ("stream") decode schedule, head dims 64/128/256, GQA group >= 4,
 // any block size. Workspace layout: part_o[2 * wgs][hpw][D],

@@ -58,23 +58,6 @@ struct StreamArgs {
   float* unit_span;       // per unit: {first partial slot, last workgroup} as int32 bits
 };
 
-// A row's tiles: visible keys [left, ctx) occupy tiles first .. first + count - 1.
-// An empty row still owns one (fully masked) tile, so every unit is finalised.
-struct RowTiles {
-  int first, count, left, ctx;
-};
-
-template <int TS>
-__device__ __forceinline__ RowTiles row_tiles(int ctx, int window) {
-  RowTiles r;
-  r.ctx = ctx > 0 ? ctx : 0;
-  r.left = visible_left(r.ctx, window);
-  r.first = r.left / TS;
-  r.count = stream_row_tile_count(r.ctx, window, TS);
-  return r;
-}
-
-
 // Inclusive prefix sum over the wave's 64 lanes with DPP lane shifts (no LDS
 // round trips): row_shr 1, 2, 4, 8 scan each 16-lane row (a source outside
 // the row reads 0), then row_bcast:15 adds row 0's total into row 1 and row

@@ -96,6 +96,9 @@ __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_ex
 constexpr float kLog2e = 1.4426950408889634f;
 
 // Launchers shared between translation units (status-returning, host side).
+// The store's checks of its source rows and pool (status-returning).
+int check_kv_store(const void* key, const void* value, int64_t key_stride, int64_t value_stride, const void* pool,
+                   int32_t kv_heads, int32_t head_dim);
 int launch_kv_store(const void* key, const void* value, int64_t key_stride, int64_t value_stride,
                     const int32_t* slot_mapping, int32_t rows, void* pool, int64_t slots, int32_t kv_heads,
                     int32_t head_dim, hipStream_t stream);

@@ -75,6 +75,15 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 
 
 }  // namespace
 
+int check_kv_store(const void* key, const void* value, int64_t key_stride, int64_t value_stride, const void* pool,
+                   int32_t kv_heads, int32_t head_dim) {
+  if (!aligned16(key) || !aligned16(value) || !aligned16(pool) || (key_stride & 7) || (value_stride & 7) ||
+      key_stride < (int64_t)kv_heads * head_dim || value_stride < (int64_t)kv_heads * head_dim)
+    return fail(GK_ERR_INVALID_ARGUMENT, "gk_kv_store: K/V rows must be 16-byte aligned and hold kv_heads * head_dim");
+  if (kv_heads > (1 << 20)) return fail(GK_ERR_INVALID_ARGUMENT, "gk_kv_store: invalid geometry");
+  return GK_OK;
+}
+
 int launch_kv_store(const void* key, const void* value, int64_t key_stride, int64_t value_stride,
                     const int32_t* slot_mapping, int32_t rows, void* pool, int64_t slots, int32_t kv_heads,
                     int32_t head_dim, hipStream_t stream) {
@@ -83,10 +92,7 @@ int launch_kv_store(const void* key, const void* value, int64_t key_stride, int6
   if (rows == 0) return GK_OK;
   if (!key || !value || !slot_mapping || !pool)
     return fail(GK_ERR_INVALID_ARGUMENT, "gk_kv_store: null pointer");
-  if (!aligned16(key) || !aligned16(value) || !aligned16(pool) || (key_stride & 7) || (value_stride & 7) ||
-      key_stride < (int64_t)kv_heads * head_dim || value_stride < (int64_t)kv_heads * head_dim)
-    return fail(GK_ERR_INVALID_ARGUMENT, "gk_kv_store: K/V rows must be 16-byte aligned and hold kv_heads * head_dim");
-  if (kv_heads > (1 << 20)) return fail(GK_ERR_INVALID_ARGUMENT, "gk_kv_store: invalid geometry");
+  if (int rc = check_kv_store(key, value, key_stride, value_stride, pool, kv_heads, head_dim)) return rc;
   const int chunk_shift = head_dim == 64 ? 3 : head_dim == 128 ? 4 : 5;
   const dim3 grid((unsigned)(((2 * kv_heads << chunk_shift) + 255) / 256), (unsigned)std::min(rows, 65535));
   kv_store_kernel<<<grid, 256, 0, stream>>>(static_cast<const uint16_t*>(key), static_cast<const uint16_t*>(value),

@@ -752,6 +752,16 @@ bool use_stream(const gk_decode_params* p) {
                           stream_decode_wgs(p->head_dim, p->softcap > 0.f, p->block_size));
 }
 
+int64_t stream_units(const gk_decode_params* p) {
+  const int group = p->q_heads / p->kv_heads;
+  const int hpw = heads_per_workgroup(group);
+  return (int64_t)p->rows * p->kv_heads * ((group + hpw - 1) / hpw);
+}
+
+// Short contexts on few units take one workgroup per unit (decode_unit.hip),
+// which needs no workspace and no merge.
+bool use_unit(const gk_decode_params* p) { return p->partition_tokens == 0 && unit_decode_fits(p, stream_units(p)); }
+
 int32_t decode_partition(const gk_decode_params* p) {
   if (p->partition_tokens > 0) return p->partition_tokens;
   if (use_stream(p)) return 0;
@@ -781,12 +791,6 @@ int32_t decode_max_parts(const gk_decode_params* p) {
   return std::max<int32_t>(1, (p->max_context + part - 1) / part);
 }
 
-int64_t stream_units(const gk_decode_params* p) {
-  const int group = p->q_heads / p->kv_heads;
-  const int hpw = heads_per_workgroup(group);
-  return (int64_t)p->rows * p->kv_heads * ((group + hpw - 1) / hpw);
-}
-
 size_t decode_workspace_bytes(const gk_decode_params* p) {
   if (p->rows > 0 && use_stream(p))
     return stream_decode_workspace_bytes(p->head_dim, heads_per_workgroup(p->q_heads / p->kv_heads), stream_units(p),
@@ -801,17 +805,24 @@ size_t decode_workspace_bytes(const gk_decode_params* p) {
 int paged_decode(const gk_decode_params* p, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   if (int rc = validate(p)) return rc;
   if (p->rows == 0) return GK_OK;
+  const bool unit = use_unit(p);
+  bool unit_store = false;
   if (p->new_key) {
     if (!p->new_value || !p->slot_mapping)
       return fail(GK_ERR_INVALID_ARGUMENT, "gk_paged_decode: fused store needs new_value and slot_mapping");
-    if (int rc = launch_kv_store(p->new_key, p->new_value, p->new_kv_row_stride, p->new_kv_row_stride,
+    unit_store = unit && p->rows <= kUnitMaxNewRows;
+    if (unit_store) {
+      if (int rc = check_kv_store(p->new_key, p->new_value, p->new_kv_row_stride, p->new_kv_row_stride, p->pool,
+                                  p->kv_heads, p->head_dim))
+        return rc;
+    } else if (int rc = launch_kv_store(p->new_key, p->new_value, p->new_kv_row_stride, p->new_kv_row_stride,
                                  p->slot_mapping, p->rows, const_cast<void*>(p->pool), p->slots, p->kv_heads,
                                  p->head_dim, stream))
       return rc;
   }
   const int32_t part = decode_partition(p);
   const int32_t max_parts = decode_max_parts(p);
-  const size_t need = decode_workspace_bytes(p);
+  const size_t need = unit ? 0 : decode_workspace_bytes(p);
   if (need > workspace_bytes || (need && !workspace))
     return fail(GK_ERR_WORKSPACE, "gk_paged_decode: workspace too small (" + std::to_string(need) + " bytes needed)");
   const int group = p->q_heads / p->kv_heads;
@@ -841,6 +852,7 @@ int paged_decode(const gk_decode_params* p, void* workspace, size_t workspace_by
   a.max_parts = max_parts;
   a.out = static_cast<uint16_t*>(p->out);
   a.out_stride = p->out_row_stride;
+  if (unit) return launch_unit_decode(a, softcap, p->head_dim, p, unit_store, stream);
   if (use_stream(p))
     return launch_stream_decode(a, softcap, p->head_dim, stream_decode_wgs(p->head_dim, softcap, p->block_size), workspace,
                                 stream);

@@ -957,8 +957,13 @@ at::Tensor paged_attn_impl(const at::Tensor& query, const at::Tensor& key, const
   auto output = bucket_output(query, plan.rows, query.size(1));
   void* pool = key_pool.data_ptr();
   // KV store first, on the same stream: rows of one sequence attend each
-  // other's new keys.
-  if (!rotary) {
+  // other's new keys. A batch of decode rows in order hands its new rows to the
+  // decode call, which stores them first or, for short contexts, along the way.
+  const bool decode_stores = !rotary && !plan.prefill_items && plan.row_context_ref.defined() &&
+                             plan.decode_rows == plan.rows && k.stride(0) == v.stride(0);
+  if (decode_stores) {
+    // below
+  } else if (!rotary) {
     check_gk(gk_kv_store(k.data_ptr(), v.data_ptr(), k.stride(0), v.stride(0), locations.data_ptr<int32_t>(),
                          static_cast<int32_t>(plan.rows), pool, plan.slots, static_cast<int32_t>(plan.kv_heads),
                          static_cast<int32_t>(head_dim), stream),
@@ -1051,6 +1056,12 @@ at::Tensor paged_attn_impl(const at::Tensor& query, const at::Tensor& key, const
     p.partition_tokens = g_decode_partition.load(std::memory_order_relaxed);
     p.out = output.data_ptr();
     p.out_row_stride = output.stride(0);
+    if (decode_stores) {
+      p.new_key = k.data_ptr();
+      p.new_value = v.data_ptr();
+      p.new_kv_row_stride = k.stride(0);
+      p.slot_mapping = locations.data_ptr<int32_t>();
+    }
     const size_t need = gk_paged_decode_workspace_bytes(&p);
     at::Tensor workspace;
     if (need) workspace = at::empty({static_cast<int64_t>(need)}, query.options().dtype(at::kByte));

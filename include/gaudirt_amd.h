@@ -87,18 +87,19 @@ typedef struct gk_decode_params {
   float softcap;               /* 0 = off */
   int32_t sliding_window;      /* <= 0 = off */
   int32_t max_context;         /* host bound: row_context[r] <= max_context for every row */
-  int32_t partition_tokens;    /* split-K partition (multiple of 32); 0 = library choice: a
+  int32_t partition_tokens;    /* split-K partition (multiple of 32); 0 = library choice: one
+                                  workgroup per (row, kv head) for short contexts, else a
                                   balanced split of all key tiles over one resident grid
                                   (any GQA group and block_size), or a partition sized from
                                   the batch for batches beyond the split's 32-bit tile
-                                  numbering; either way a row's split points,
+                                  numbering; in each case a row's split points,
                                   and so its last bits, depend on the whole batch. A fixed
                                   partition (> 0) makes every row's output a function of
                                   that row alone, bit for bit (batch-invariant decode) */
   void* out;                   /* bf16 [rows, out_row_stride] */
   int64_t out_row_stride;      /* elements */
   /* Optional fused KV store of the new token rows (NULL new_key = none): written
-   * with gk_kv_store semantics before any key is read. */
+   * with gk_kv_store semantics, as if before any key is read. */
   const void* new_key;
   const void* new_value;
   int64_t new_kv_row_stride;
@@ -111,7 +112,9 @@ typedef struct gk_decode_params {
 /* Workspace bytes gk_paged_decode needs for these parameters (0 if none). */
 size_t gk_paged_decode_workspace_bytes(const gk_decode_params* params);
 /* The split-K partition gk_paged_decode uses for these parameters; 0 when the
- * balanced split (partitions chosen on the device from row_context) applies. */
+ * balanced split (partitions chosen on the device from row_context) or, for
+ * short contexts, one workgroup per unit applies (the latter leaves the
+ * workspace untouched). */
 int32_t gk_paged_decode_partition_tokens(const gk_decode_params* params);
 int gk_paged_decode(const gk_decode_params* params, void* workspace, size_t workspace_bytes,
                     hipStream_t stream);
