@@ -76,13 +76,23 @@ __global__ __launch_bounds__(kUnitWaves * 64, 1) void decode_unit_kernel(UnitArg
   // The row's block-table entries of its visible keys, its query and its new
   // K/V row: one memory round trip.
   const int e0 = rt.left >> shift, ne = rt.ctx > 0 ? ((rt.ctx - 1) >> shift) - e0 + 1 : 0;
-  if (ne > unit_max_keys(D) + 1) {
-    // A caller whose row_context exceeds its max_context.
-    for (int e = tid; e < hv * D; e += kUnitWaves * 64) out[e] = 0x7fc0;
-    return;
-  }
+  // A row_context beyond the caller's max_context (a graph replayed on longer
+  // rows) may need more entries than LDS holds: they are then read in place.
+  constexpr int kEntries = unit_max_keys(D) + 1;
+  const bool in_lds = ne <= kEntries;
   const int32_t* bt = a.block_tables + (int64_t)request * a.bt_stride + e0;
-  for (int i = tid; i < ne; i += kUnitWaves * 64) s_bt[i] = bt[i];
+  for (int i = tid; i < min(ne, kEntries); i += kUnitWaves * 64) s_bt[i] = bt[i];
+  auto entries_at = [&](int32_t* e, const int* i, auto n) __attribute__((always_inline)) {
+    if (in_lds) {
+#pragma unroll
+      for (int k = 0; k < n; ++k) e[k] = s_bt[i[k]];
+    } else {
+#pragma unroll
+      for (int k = 0; k < n; ++k) e[k] = bt[i[k]];
+#pragma unroll
+      for (int k = 0; k < n; ++k) asm volatile("" : "+v"(e[k]));  // waited for here, not where the branches meet
+    }
+  };
   bf16x8_t qb[S::NC];
   {
     const uint16_t* src = a.query + (int64_t)qrow * a.q_stride + (int64_t)(head0 + c16) * D;
@@ -126,11 +136,16 @@ __global__ __launch_bounds__(kUnitWaves * 64, 1) void decode_unit_kernel(UnitArg
   };
   auto offsets_of = [&](int tb) __attribute__((always_inline)) {
     Offsets of;
+    int32_t e[LOADS];
+    int at[LOADS];
+    const auto key_of = [&](int i) { return min(max(tb + (i * 64 + lane) / CPR, rt.left), rt.ctx - 1); };
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) at[i] = (key_of(i) >> shift) - e0;
+    entries_at(e, at, std::integral_constant<int, LOADS>{});
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
       const int s = i * 64 + lane, tt = s / CPR, pc = s % CPR;
-      const int key = min(max(tb + tt, rt.left), rt.ctx - 1);
-      const uint32_t slot = ((uint32_t)s_bt[(key >> shift) - e0] << shift) | (uint32_t)(key & bmask);
+      const uint32_t slot = ((uint32_t)e[i] << shift) | (uint32_t)(key_of(i) & bmask);
       of.v[i] = slot * (uint32_t)(2 * D) + ((pc ^ swz(tt, D / 8)) << 4);
     }
     return of;
@@ -147,7 +162,9 @@ __global__ __launch_bounds__(kUnitWaves * 64, 1) void decode_unit_kernel(UnitArg
   auto new_row_of = [&](int tb) __attribute__((always_inline)) {
     const int key = tb + (lane & (TS - 1));
     const bool visible = key >= rt.left && key < rt.ctx;
-    const int entry = s_bt[(min(max(key, rt.left), rt.ctx - 1) >> shift) - e0];
+    const int at = (min(max(key, rt.left), rt.ctx - 1) >> shift) - e0;
+    int32_t entry;
+    entries_at(&entry, &at, std::integral_constant<int, 1>{});
     const int slot = visible && entry >= 0 ? (int)(((uint32_t)entry << shift) | (uint32_t)(key & bmask)) : kNoKey;
     const int g0 = (lane / TS) * share;
     int found = -1;

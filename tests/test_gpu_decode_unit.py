@@ -117,8 +117,9 @@ def test_window_inside_a_page_at_the_limit(runner):
     step(runner, 4, 1, 128, 1, [3001, 2500], window=2048)
 
 
-def test_contexts_beyond_max_context_give_nan(runner):
-    # row_context above the caller's bound: no read past the entries' LDS, NaN rows instead.
+def test_contexts_beyond_max_context(runner):
+    # A graph replayed on rows that outgrew its max_context: more block-table
+    # entries than the workgroup keeps in LDS.
     import torch
 
     case = cases.decode_case(5, 2, 4, 1, 128, 1, 6000, [2800, 100])
@@ -129,4 +130,4 @@ def test_contexts_beyond_max_context_give_nan(runner):
     ws = runner.paged_decode(params)
     torch.cuda.synchronize()
     del ws
-    assert torch.isnan(out[0].float()).all() and torch.isfinite(out[1].float()).all()
+    orc.check_tolerance(runner.bits_of(out), orc.direct_bf16_pv(case.oracle_problem()), MAX_ABS, MEAN_ABS)
