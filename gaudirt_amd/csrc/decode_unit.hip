@@ -226,6 +226,7 @@ __global__ __launch_bounds__(kUnitWaves * 64, 1) void decode_unit_kernel(UnitArg
 #pragma unroll
       for (int c = 0; c < S::NC; ++c) sc[g] = mfma32(kr[g][c], qb[c], sc[g]);
     }
+    mfma_results_ready(sc);
     const bool inside = !SOFTCAP && tb >= rt.left && tb + TS <= rt.ctx;
     if (!inside) {
 #pragma unroll

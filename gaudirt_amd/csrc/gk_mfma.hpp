@@ -81,6 +81,19 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
   asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
+// The wait states between an MFMA and a read of its result by inline asm (max2,
+// max3): a matrix result reaches the registers several issue slots later, the
+// compiler counts them for its own instructions only, and asm that comes sooner
+// reads the value before the last accumulation. Needed where the maxima can
+// follow the MFMAs directly, with no compiler-visible instruction on the scores
+// or a dozen others between.
+template <int N>
+__device__ __forceinline__ void mfma_results_ready(f32x4_t (&x)[N]) {
+  static_assert(N == 1 || N == 2, "one or two tiles");
+  if constexpr (N == 1) asm volatile("s_nop 15" : "+v"(x[0]));
+  else asm volatile("s_nop 15" : "+v"(x[0]), "+v"(x[1]));
+}
+
 // Maximum of N >= 2 values as a tree of bare max3 (depth log3 N): a chain
 // would be N / 2 dependent instructions, and fmaxf would quiet every input
 // first.

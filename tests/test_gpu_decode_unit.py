@@ -63,6 +63,10 @@ def step(runner, heads, kv_heads, d, block, lens, requests=None, softcap=0.0, wi
     assert np.array_equal(runner.bits_of(pool), expected), "KV store differs from the oracle"
     actual = runner.bits_of(out)
     assert np.isfinite(orc.bf16_to_f32(actual)).all()
+    for _ in range(3):
+        runner.paged_decode(params)
+        torch.cuda.synchronize()
+        assert np.array_equal(runner.bits_of(out), actual), "the same step twice gives other bits"
     mapping = orc.mapping_from_block_table(case.block_tables, block, int(longest.max()))
     live = np.flatnonzero(lens > 0)
     problem = orc.Problem(query[live], expected, requests[live], positions[live].astype(np.int64), mapping, heads,

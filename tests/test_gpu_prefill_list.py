@@ -90,3 +90,14 @@ def test_split_items(heads, kv_heads, d, block, prefixes, chunks, softcap, windo
     assert np.isfinite(orc.bf16_to_f32(actual)).all()
     max_abs, mean_abs = orc.check_tolerance(actual, reference, MAX_ABS, MEAN_ABS)
     print(f"items={lst.item_count} merges={lst.merge_count} max_abs={max_abs:.3e} mean_abs={mean_abs:.3e}", flush=True)
+
+
+@pytest.mark.parametrize("heads,kv_heads,d", [(16, 8, 256), (32, 8, 128), (14, 2, 64)])
+def test_repeats_are_bit_identical(heads, kv_heads, d):
+    # Every product of a step has to be complete before the step's maxima read
+    # it: a maximum taken too early gives another base, and other last bits from
+    # run to run.
+    case = cases.PrefillCase(d, heads, kv_heads, d, 16, prefixes=[1500, 300], chunks=[300, 200])
+    first, _ = run(case, -1)
+    for _ in range(4):
+        assert np.array_equal(run(case, -1)[0], first)
