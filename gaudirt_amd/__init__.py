@@ -56,6 +56,7 @@ def load_extension():
             f"({exc})") from exc
     from . import _C as ext
     _register_fakes(torch)
+    _call_directly(torch)
     _ext = ext
     env = os.environ.get("GAUDIRT_AMD_BATCH_INVARIANT_DECODE", "").strip()
     if env and env != "0":
@@ -73,6 +74,38 @@ def set_batch_invariant_decode(enabled=True, partition_tokens=BATCH_INVARIANT_PA
 def batch_invariant_decode():
     """The fixed decode partition in keys, or 0 when the library chooses."""
     return load_extension()._decode_partition()
+
+
+def _call_directly(torch):
+    """Calls of the metadata operators without torch's per-call search for fake script objects.
+
+    For an operator with a custom-class argument, ``torch.ops.gaudirt.op(...)``
+    looks through all call arguments, as a tree, for the stand-ins that export
+    and fake tracing use: 6 us of the 18.7 us of a small attention call. These
+    operators have exactly one such argument, the metadata; when it is the real
+    object the search finds nothing and the registered operator is called next,
+    which is all that happens here. Every other call (metadata by keyword, a
+    stand-in, too few arguments) takes torch's own path, as do the overloads
+    (``.default``) and all calls on a torch that keeps its operators elsewhere.
+    """
+    real = torch.ScriptObject
+
+    def direct(base, position):
+        class Direct(base):
+            __slots__ = ()
+
+            def __call__(self, /, *args, **kwargs):
+                if len(args) > position and type(args[position]) is real:
+                    return self._op(*args, **kwargs)
+                return base.__call__(self, *args, **kwargs)
+
+        Direct.__name__, Direct.__qualname__, Direct.__module__ = base.__name__, base.__qualname__, base.__module__
+        return Direct
+
+    for name, position in (("paged_attn", 5), ("rotary_paged_attn", 6), ("rotary_embedding", 3)):
+        packet = getattr(torch.ops.gaudirt, name)
+        if callable(getattr(packet, "_op", None)):
+            packet.__class__ = direct(type(packet), position)
 
 
 def _register_fakes(torch):
