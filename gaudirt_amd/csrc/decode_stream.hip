@@ -933,11 +933,14 @@ struct StreamMergeArgs {
   int64_t out_stride;
 };
 
-// One wave per (row, query head).
-template <int D>
-__global__ __launch_bounds__(64) void stream_merge_kernel(StreamMergeArgs m) {
+// One workgroup per (row, query head): one wave, or kMergeWaves that take a run
+// of the unit's parts each and meet in LDS.
+constexpr int kMergeWaves = 8;
+template <int D, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void stream_merge_kernel(StreamMergeArgs m) {
   constexpr int PER_LANE = D / 64;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63;
+  const int wave = WAVES > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) : 0;
   const int head = blockIdx.x, row = blockIdx.y;
   const int kvh = head / m.group, within = head - kvh * m.group;
   const int hg = within / 16, hh = within - hg * 16;
@@ -957,13 +960,15 @@ __global__ __launch_bounds__(64) void stream_merge_kernel(StreamMergeArgs m) {
   float acc[PER_LANE];
 #pragma unroll
   for (int e = 0; e < PER_LANE; ++e) acc[e] = 0.f;
+  // This wave's parts [first, end).
+  const int run = (nslots + WAVES - 1) / WAVES, first = wave * run, end = min(first + run, nslots);
   auto merge_parts = [&](auto batch) {
     constexpr int BATCH = decltype(batch)::value;
-    for (int k0 = 0; k0 < nslots; k0 += BATCH) {
+    for (int k0 = first; k0 < end; k0 += BATCH) {
       float mp[BATCH], lp[BATCH], op[BATCH][PER_LANE];
 #pragma unroll
       for (int u = 0; u < BATCH; ++u) {
-        const int64_t pi = (int64_t)slot_of_part(min(k0 + u, nslots - 1)) * m.heads_per_group + hh;
+        const int64_t pi = (int64_t)slot_of_part(min(k0 + u, end - 1)) * m.heads_per_group + hh;
         mp[u] = m.part_ml[pi * 2];
         lp[u] = m.part_ml[pi * 2 + 1];
 #pragma unroll
@@ -971,8 +976,8 @@ __global__ __launch_bounds__(64) void stream_merge_kernel(StreamMergeArgs m) {
       }
 #pragma unroll
       for (int u = 0; u < BATCH; ++u) {
-        // Slots past the unit's last (clamped duplicates) weigh zero.
-        const float mu = k0 + u < nslots ? mp[u] : -INFINITY;
+        // Slots past the run's last (clamped duplicates) weigh zero.
+        const float mu = k0 + u < end ? mp[u] : -INFINITY;
         const float mn = fmaxf(mm, mu);
         const float fa = mm == -INFINITY ? 0.f : fast_exp2(mm - mn);
         const float fb = mu == -INFINITY ? 0.f : fast_exp2(mu - mn);
@@ -983,8 +988,32 @@ __global__ __launch_bounds__(64) void stream_merge_kernel(StreamMergeArgs m) {
       }
     }
   };
-  if (nslots <= 4) merge_parts(std::integral_constant<int, 4>{});
+  if (run <= 4) merge_parts(std::integral_constant<int, 4>{});
   else merge_parts(std::integral_constant<int, 16>{});
+  if constexpr (WAVES > 1) {
+    __shared__ float s_m[WAVES], s_l[WAVES], s_o[WAVES][D];
+    if (lane == 0) {
+      s_m[wave] = mm;
+      s_l[wave] = ll;
+    }
+#pragma unroll
+    for (int e = 0; e < PER_LANE; ++e) s_o[wave][lane + 64 * e] = acc[e];
+    __syncthreads();
+    if (wave) return;
+    mm = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) mm = fmaxf(mm, s_m[w]);
+    ll = 0.f;
+#pragma unroll
+    for (int e = 0; e < PER_LANE; ++e) acc[e] = 0.f;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float f = s_m[w] == -INFINITY ? 0.f : fast_exp2(s_m[w] - mm);
+      ll += s_l[w] * f;
+#pragma unroll
+      for (int e = 0; e < PER_LANE; ++e) acc[e] += s_o[w][lane + 64 * e] * f;
+    }
+  }
   const float inv = ll > 0.f ? 1.f / ll : 0.f;
   const int orow = m.row_map ? m.row_map[row] : row;
   uint16_t* dst = m.out + (int64_t)orow * m.out_stride + (int64_t)head * D;
@@ -1114,11 +1143,22 @@ int launch_stream_decode(const DecodeArgs& a, bool softcap, int head_dim, int wg
   m.out = a.out;
   m.out_stride = a.out_stride;
   const dim3 mgrid(a.q_heads, a.rows);
-  switch (head_dim) {
-    case 64: stream_merge_kernel<64><<<mgrid, 64, 0, stream>>>(m); break;
-    case 128: stream_merge_kernel<128><<<mgrid, 64, 0, stream>>>(m); break;
-    default: stream_merge_kernel<256><<<mgrid, 64, 0, stream>>>(m); break;
-  }
+  const auto merge = [&](auto waves) {
+    constexpr int W = decltype(waves)::value;
+    switch (head_dim) {
+      case 64: stream_merge_kernel<64, W><<<mgrid, 64 * W, 0, stream>>>(m); break;
+      case 128: stream_merge_kernel<128, W><<<mgrid, 64 * W, 0, stream>>>(m); break;
+      default: stream_merge_kernel<256, W><<<mgrid, 64 * W, 0, stream>>>(m); break;
+    }
+  };
+  // Few (row, head) pairs have their parts from many workgroups each (one row of
+  // 8 kv heads: 128): a single wave walks them sixteen to a round trip, most of
+  // the GPU idle. Whole step, one wave / eight (us): 1 row x 32 heads, 16384 keys
+  // 32.2 / 22.4; 1 x 14 (head_dim 64), 32768 keys 62.8 / 20.5; 8 x 32, 8192 keys
+  // 50.7 / 50.2; 16 x 32 50.7 / 50.3 (4096); from 1024 pairs on the extra waves
+  // only cost: 16 x 64, 4096 keys 51.1 / 51.6; 32 x 64 90.4 / 92.4.
+  if ((int64_t)a.rows * a.q_heads <= 512) merge(std::integral_constant<int, kMergeWaves>{});
+  else merge(std::integral_constant<int, 1>{});
   return hip_status(hipGetLastError(), "gk_paged_decode stream merge launch");
 }
 
