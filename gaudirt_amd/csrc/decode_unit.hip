@@ -351,19 +351,22 @@ __global__ __launch_bounds__(kUnitWaves * 64, 1) void decode_unit_kernel(UnitArg
 
 // Where one workgroup per unit is the faster form, by time on the stream, both
 // with the fused store (us; balanced schedule / unit kernel):
-//   head_dim 128, 8 units x 512 keys 11.3 / 7.8, x 2048 17.5 / 17.2, x 3072
-//   20.9 / 23.0; 256 units x 2048 51.9 / 42.1, x 3072 71.2 / 72.4; 512 units x
-//   64 14.3 / 9.8, x 1024 50.6 / 44.0, x 1536 69.0 / 74.1; 1024 units x 64
-//   14.9 / 19.7.
-//   head_dim 64, 8 x 2048 15.6 / 11.9; 256 x 4096 51.2 / 42.4; 512 x 2048
-//   52.4 / 42.9, x 3072 72.2 / 73.1. head_dim 256, 8 x 1024 21.7 / 18.1, x 1536
-//   20.2 / 24.2; 256 x 1024 51.0 / 42.2; 512 x 512 51.8 / 43.6, x 1024 90.6 /
-//   95.9.
-// So: at most 1 MiB of keys and values a unit (a CU streams it in 12-17 us) and
-// 256 MiB in all, and at most two rounds of workgroups.
+//   head_dim 128, 8 units x 64 keys 10.5 / 5.0, x 512 10.8 / 7.5, x 1024 10.8 /
+//   10.6, x 1536 12.3 / 13.5, x 2048 12.6 / 16.5; 64 units x 2048 21.1 / 17.5;
+//   256 x 512 21.0 / 13.9, x 2048 51.4 / 42.2, x 3072 71.2 / 72.4; 512 x 64
+//   14.3 / 9.8, x 1024 50.6 / 44.0, x 1536 69.0 / 74.1; 1024 x 64 14.9 / 19.7.
+//   head_dim 64, 8 x 2048 11.0 / 11.7, x 3000 11.5 / 15.5; 256 x 3000 40.0 /
+//   32.6; 512 x 2048 52.4 / 42.9, x 3072 72.2 / 73.1. head_dim 256, 8 x 512
+//   11.0 / 10.9, x 768 13.5 / 14.0, x 1024 14.0 / 16.6; 256 x 1024 50.8 / 43.5;
+//   512 x 512 51.8 / 43.6, x 1024 90.6 / 95.9.
+// So: at most 1 MiB of keys and values a unit and 256 MiB in all, and at most
+// two rounds of workgroups; 3/4 MiB (2048 keys) where fewer than 32 units leave
+// the GPU to the balanced schedule's many workgroups. Up to 2 us of stream time
+// are given for the two launches (7 us of host time) that the unit form saves.
 bool unit_decode_fits(const gk_decode_params* p, int64_t units) {
   const int64_t visible = p->sliding_window > 0 ? std::min(p->max_context, p->sliding_window) : p->max_context;
-  return visible <= unit_max_keys(p->head_dim) && units <= 512 && units * visible * p->head_dim <= int64_t(1) << 26;
+  const int64_t most = units < 32 ? std::min(2048, (3 << 16) / p->head_dim) : unit_max_keys(p->head_dim);
+  return visible <= most && units <= 512 && units * visible * p->head_dim <= int64_t(1) << 26;
 }
 
 int launch_unit_decode(const DecodeArgs& a, bool softcap, int head_dim, const gk_decode_params* p, bool store,

@@ -109,16 +109,19 @@ def test_row_counts(runner, rows):
     step(runner, 4, 1, 64, 1, rng.integers(1, 130, rows), seed=rows)
 
 
-@pytest.mark.parametrize("d,longest", [(64, 3072), (64, 3073), (128, 2048), (128, 2049), (256, 1024), (256, 1025)])
+@pytest.mark.parametrize("d,few,many", [(64, 2048, 3072), (128, 1536, 2048), (256, 768, 1024)])
 @pytest.mark.parametrize("block", [1, 32])
-def test_lengths_around_the_rule(runner, d, longest, block):
-    step(runner, 4, 1, d, block, [longest, longest - 33, 7])
+@pytest.mark.parametrize("above", [0, 1])
+def test_lengths_around_the_rule(runner, d, few, many, block, above):
+    # Fewer than 32 units and 32: each longest row on both sides of its limit.
+    step(runner, 4, 1, d, block, [few + above, few - 33, 7])
+    step(runner, 4, 1, d, block, [many + above, many - 33] + [5] * 30)
 
 
 def test_window_inside_a_page_at_the_limit(runner):
     # 2048 visible keys that start inside a page: one block-table entry more than keys / page.
-    step(runner, 4, 1, 128, 16, [3001, 2500], window=2048)
-    step(runner, 4, 1, 128, 1, [3001, 2500], window=2048)
+    step(runner, 4, 1, 128, 16, [3001, 2500] + [9] * 30, window=2048)
+    step(runner, 4, 1, 128, 1, [3001, 2500] + [9] * 30, window=2048)
 
 
 def test_contexts_beyond_max_context(runner):
