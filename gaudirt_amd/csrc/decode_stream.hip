@@ -654,7 +654,7 @@ __device__ __forceinline__ void decode_stream_body(StreamArgs sa) {
       const float part = a0 + a1;
       const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(part), __float_as_uint(part), false, false);
       float sv = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-      if constexpr (SOFTCAP) sv = a.softcap_log2 * soft_tanh(sv * a.score_scale);
+      if constexpr (SOFTCAP) sv = soft_cap(sv * a.score_scale, a.softcap_log2);
       const int k = t.tb + key;
       sd[h] = (SOFTCAP || !(t.tb >= t.left && t.tb + TS <= t.ctx)) ? ((k >= t.left && k < t.ctx) ? sv : -INFINITY)
                                                                     : sv;
@@ -775,7 +775,7 @@ __device__ __forceinline__ void decode_stream_body(StreamArgs sa) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           float s = sc[h][r];
-          if constexpr (SOFTCAP) s = a.softcap_log2 * soft_tanh(s * a.score_scale);
+          if constexpr (SOFTCAP) s = soft_cap(s * a.score_scale, a.softcap_log2);
           const int key = t.tb + 16 * h + 4 * q + r;
           sc[h][r] = (key >= t.left && key < t.ctx) ? s : -INFINITY;
         }

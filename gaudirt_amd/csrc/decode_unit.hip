@@ -234,7 +234,7 @@ __global__ __launch_bounds__(kUnitWaves * 64, 1) void decode_unit_kernel(UnitArg
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
           float s = sc[g][r];
-          if constexpr (SOFTCAP) s = a.softcap_log2 * soft_tanh(s * a.score_scale);
+          if constexpr (SOFTCAP) s = soft_cap(s * a.score_scale, a.softcap_log2);
           const int key = tb + 16 * g + 4 * q + r;
           sc[g][r] = (key >= rt.left && key < rt.ctx) ? s : -INFINITY;
         }

@@ -230,7 +230,7 @@ __global__ __launch_bounds__(64, mfma_waves_per_simd<D>()) void decode_mfma_kern
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         float s;
-        if constexpr (SOFTCAP) s = a.softcap_log2 * soft_tanh(sc[h][r] * a.score_scale);
+        if constexpr (SOFTCAP) s = soft_cap(sc[h][r] * a.score_scale, a.softcap_log2);
         else s = sc[h][r] * a.score_scale;
         s = (tb + 16 * h + 4 * q + r < pr.t_end) ? s : -INFINITY;
         sc[h][r] = s;
@@ -459,7 +459,7 @@ __global__ __launch_bounds__(kWaves * 64) void decode_dot_kernel(DecodeArgs a) {
         }
         acc = group_sum<LPT>(acc);
         float s;
-        if constexpr (SOFTCAP) s = a.softcap_log2 * soft_tanh(acc * a.score_scale);
+        if constexpr (SOFTCAP) s = soft_cap(acc * a.score_scale, a.softcap_log2);
         else s = acc * a.score_scale;
         p[u][gh] = valid[u] ? s : -INFINITY;
       }

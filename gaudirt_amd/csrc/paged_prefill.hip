@@ -451,7 +451,7 @@ __global__ __launch_bounds__(kPrefillWaves * 64, 1) void prefill_kernel(PrefillA
   // place (the same registers on both paths), the row maximum is taken on raw
   // scores (scale > 0), and p = exp2(fma(s, scale, -max)).
   auto softmax = [&](int tb) __attribute__((always_inline)) {
-    const bool full = !SOFTCAP && tb + kKeys - 1 <= wave_pos_min && tb >= wave_left_max;
+    const bool full = tb + kKeys - 1 <= wave_pos_min && tb >= wave_left_max;
     // At head_dim 256 the maxima can come two issue slots after the scores (at
     // 128 the early V reads lie between, at 64 the P.V products and a barrier).
     if constexpr (D == 256 && !SOFTCAP) {
@@ -468,12 +468,9 @@ __global__ __launch_bounds__(kPrefillWaves * 64, 1) void prefill_kernel(PrefillA
 #pragma unroll
         for (int h = 0; h < kKG; ++h)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int key = tb + 16 * h + 4 * q + r;
-            const float sv = a.softcap_log2 * soft_tanh(sc[h][nt][r] * a.score_scale);
-            sc[h][nt][r] = (key <= qpos[nt] && key >= qleft[nt]) ? sv : -INFINITY;
-          }
-      } else if (!full) {
+          for (int r = 0; r < 4; ++r) sc[h][nt][r] = soft_cap(sc[h][nt][r] * a.score_scale, a.softcap_log2);
+      }
+      if (!full) {
 #pragma unroll
         for (int h = 0; h < kKG; ++h)
 #pragma unroll
