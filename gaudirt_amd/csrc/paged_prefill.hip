@@ -566,6 +566,27 @@ __global__ __launch_bounds__(kPrefillWaves * 64, 1) void prefill_kernel(PrefillA
       issue(first, vrs, kv[0][1]);
     }
     if (1 < nsteps) e_next = entry_of(kb0 + kKeys);
+    if (__builtin_expect(div_group(wave * kQrowsPerWave) >= nr, 0)) {
+      // All rows of this wave lie past the tile's last: it only loads its share
+      // and keeps step, and the other wave of its SIMD has the matrix cores and
+      // the LDS to itself (256 workgroups of 64 steps, half the waves active:
+      // head_dim 128 113.9 -> 82.6 us, with softcap 189.8 -> 120.0; three
+      // quarters 116.6 -> 110.6. A branch inside the loop below instead cost full
+      // tiles 2%).
+      for (int step = 0; step < nsteps; ++step) {
+        wait_vmem<0>();
+        __syncthreads();
+        wait_vmem_visible();
+        if (step + 1 < nsteps) {
+          const int tb = kb0 + step * kKeys, next = (step + 1) & 1;
+          const Offsets of = offsets_of(tb + kKeys, e_next);
+          issue(of, krs, kv[next][0]);
+          issue(of, vrs, kv[next][1]);
+          if (step + 2 < nsteps) e_next = entry_of(tb + 2 * kKeys);
+        }
+      }
+      return;
+    }
     // The loop is unrolled over the two stages, so that every LDS address of a
     // step is a per-lane offset plus an immediate (stage, 16-key group, half):
     // ~44 fewer VALU instructions per wave and step (C4: 148.6 -> 138.0 us).
