@@ -72,6 +72,7 @@ __device__ __forceinline__ RowTiles row_tiles(int ctx, int window) {
 // a CU's LDS), whose block-table entries, one more when a window starts inside
 // a page, lie in LDS; and as many new rows with a fused store.
 constexpr int unit_max_keys(int head_dim) { return head_dim == 64 ? 3072 : (1 << 18) / head_dim; }
+constexpr int unit_short_keys(int waves) { return 128 * waves; }  // with fewer than eight waves
 constexpr int kUnitMaxNewRows = 256;
 bool unit_decode_fits(const gk_decode_params* params, int64_t units);
 int launch_unit_decode(const DecodeArgs& a, bool softcap, int head_dim, const gk_decode_params* params, bool store,

@@ -33,7 +33,6 @@
 namespace gk {
 namespace {
 
-constexpr int kUnitWaves = 8;
 // In place of a slot where there is none: a new row that is not stored, a key
 // that is not visible.
 constexpr int32_t kNoSlot = INT32_MIN, kNoKey = -1;
@@ -50,15 +49,17 @@ struct UnitArgs {
   const int32_t* slot_mapping;
 };
 
-template <int D, bool SOFTCAP>
-__global__ __launch_bounds__(kUnitWaves * 64, 1) void decode_unit_kernel(UnitArgs ua) {
+// WAVES: 8, or fewer for short rows of many units (unit_waves).
+template <int D, bool SOFTCAP, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 1) void decode_unit_kernel(UnitArgs ua) {
   using S = MfmaShape<D>;
   constexpr int TS = S::TS, LOADS = S::LOADS, CPR = S::CPR;
   static_assert(16 * D * 4 <= 2 * S::TILE, "a wave's partial output fits its stage");
-  __shared__ __attribute__((aligned(16))) char stage[kUnitWaves][2][S::TILE];
-  __shared__ int32_t s_bt[unit_max_keys(D) + 1];
+  __shared__ __attribute__((aligned(16))) char stage[WAVES][2][S::TILE];
+  constexpr int kEntries = (WAVES < 8 ? unit_short_keys(WAVES) : unit_max_keys(D)) + 1;
+  __shared__ int32_t s_bt[kEntries];
   __shared__ __attribute__((aligned(16))) int32_t s_new[kUnitMaxNewRows];
-  __shared__ float s_m[kUnitWaves][16], s_l[kUnitWaves][16];
+  __shared__ float s_m[WAVES][16], s_l[WAVES][16];
 
   const DecodeArgs& a = ua.d;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -78,10 +79,9 @@ __global__ __launch_bounds__(kUnitWaves * 64, 1) void decode_unit_kernel(UnitArg
   const int e0 = rt.left >> shift, ne = rt.ctx > 0 ? ((rt.ctx - 1) >> shift) - e0 + 1 : 0;
   // A row_context beyond the caller's max_context (a graph replayed on longer
   // rows) may need more entries than LDS holds: they are then read in place.
-  constexpr int kEntries = unit_max_keys(D) + 1;
   const bool in_lds = ne <= kEntries;
   const int32_t* bt = a.block_tables + (int64_t)request * a.bt_stride + e0;
-  for (int i = tid; i < min(ne, kEntries); i += kUnitWaves * 64) s_bt[i] = bt[i];
+  for (int i = tid; i < min(ne, kEntries); i += WAVES * 64) s_bt[i] = bt[i];
   auto entries_at = [&](int32_t* e, const int* i, auto n) __attribute__((always_inline)) {
     if (in_lds) {
 #pragma unroll
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(kUnitWaves * 64, 1) void decode_unit_kernel(UnitArg
   };
   u32x4_t own{0u, 0u, 0u, 0u};
   if (ua.new_key) {
-    for (int s = tid; s < kUnitMaxNewRows; s += kUnitWaves * 64) {
+    for (int s = tid; s < kUnitMaxNewRows; s += WAVES * 64) {
       const int slot = s < a.rows ? ua.slot_mapping[s] : -1;
       s_new[s] = slot >= 0 && slot < a.slots ? slot : kNoSlot;
     }
@@ -189,10 +189,10 @@ __global__ __launch_bounds__(kUnitWaves * 64, 1) void decode_unit_kernel(UnitArg
     issue(next, krs, kt);
     issue(next, vrs, vt);
   }
-  for (int k = wave; k < ntiles; k += kUnitWaves) {
+  for (int k = wave; k < ntiles; k += WAVES) {
     const int tb = (rt.first + k) * TS;
-    const bool more = k + kUnitWaves < ntiles;
-    if (more) next = offsets_of(tb + kUnitWaves * TS);
+    const bool more = k + WAVES < ntiles;
+    if (more) next = offsets_of(tb + WAVES * TS);
     const int found = share ? new_row_of(tb) : -1;
     uint64_t hits = __builtin_amdgcn_ballot_w64(found >= 0);
     if (hits) {
@@ -323,14 +323,14 @@ __global__ __launch_bounds__(kUnitWaves * 64, 1) void decode_unit_kernel(UnitArg
       for (int c = 0; c < S::NO; ++c) po[(4 * q + r) * D + 16 * c + c16] = o[c][r];
     }
   __syncthreads();
-  for (int idx = tid; idx < hv * D; idx += kUnitWaves * 64) {
+  for (int idx = tid; idx < hv * D; idx += WAVES * 64) {
     const int hh = idx / D;
     float mm = -INFINITY;
 #pragma unroll
-    for (int w = 0; w < kUnitWaves; ++w) mm = fmaxf(mm, s_m[w][hh]);
+    for (int w = 0; w < WAVES; ++w) mm = fmaxf(mm, s_m[w][hh]);
     float acc = 0.f, ll = 0.f;
 #pragma unroll
-    for (int w = 0; w < kUnitWaves; ++w) {
+    for (int w = 0; w < WAVES; ++w) {
       const float f = s_m[w][hh] == -INFINITY ? 0.f : fast_exp2(s_m[w][hh] - mm);
       ll += s_l[w][hh] * f;
       acc += reinterpret_cast<const float*>(stage[w][0])[idx] * f;
@@ -338,7 +338,7 @@ __global__ __launch_bounds__(kUnitWaves * 64, 1) void decode_unit_kernel(UnitArg
     out[idx] = (uint16_t)bf16_bits(acc * (ll > 0.f ? 1.f / ll : 0.f));
   }
   // The row's new key and value, by the last wave of the kv head's first unit.
-  if (ua.new_key && hg == 0 && wave == kUnitWaves - 1) {
+  if (ua.new_key && hg == 0 && wave == WAVES - 1) {
     const int slot = s_new[row];
     if (slot != kNoSlot && lane < 2 * CPR) {
       uint16_t* dst = a.pool_out + ((int64_t)(key_lane ? kvh : a.kv_heads + kvh) * a.slots + slot) * D + chunk * 8;
@@ -349,25 +349,58 @@ __global__ __launch_bounds__(kUnitWaves * 64, 1) void decode_unit_kernel(UnitArg
 
 }  // namespace
 
-// Where one workgroup per unit is the faster form, by time on the stream, both
-// with the fused store (us; balanced schedule / unit kernel):
+// Where one workgroup per unit is the faster form, and with how many waves, by
+// time on the stream, both with the fused store (us; balanced schedule / unit
+// kernel):
 //   head_dim 128, 8 units x 64 keys 10.5 / 5.0, x 512 10.8 / 7.5, x 1024 10.8 /
 //   10.6, x 1536 12.3 / 13.5, x 2048 12.6 / 16.5; 64 units x 2048 21.1 / 17.5;
-//   256 x 512 21.0 / 13.9, x 2048 51.4 / 42.2, x 3072 71.2 / 72.4; 512 x 64
-//   14.3 / 9.8, x 1024 50.6 / 44.0, x 1536 69.0 / 74.1; 1024 x 64 14.9 / 19.7.
+//   256 x 512 21.0 / 13.9, x 2048 51.4 / 42.2, x 3072 71.2 / 72.4; 512 x 1024
+//   50.6 / 44.0, x 1536 69.0 / 74.1.
 //   head_dim 64, 8 x 2048 11.0 / 11.7, x 3000 11.5 / 15.5; 256 x 3000 40.0 /
 //   32.6; 512 x 2048 52.4 / 42.9, x 3072 72.2 / 73.1. head_dim 256, 8 x 512
 //   11.0 / 10.9, x 768 13.5 / 14.0, x 1024 14.0 / 16.6; 256 x 1024 50.8 / 43.5;
 //   512 x 512 51.8 / 43.6, x 1024 90.6 / 95.9.
-// So: at most 1 MiB of keys and values a unit and 256 MiB in all, and at most
-// two rounds of workgroups; 3/4 MiB (2048 keys) where fewer than 32 units leave
-// the GPU to the balanced schedule's many workgroups. Up to 2 us of stream time
-// are given for the two launches (7 us of host time) that the unit form saves.
-bool unit_decode_fits(const gk_decode_params* p, int64_t units) {
+// So eight waves for at most 1 MiB of keys and values a unit, 256 MiB in all and
+// 512 units; 3/4 MiB (2048 keys) where fewer than 32 units leave the GPU to the
+// balanced schedule's many workgroups. Up to 2 us of stream time are given for
+// the two launches (7 us of host time) that the unit form saves.
+// More units than CUs hold of the eight-wave form (one a CU; two at head_dim 64)
+// run in rounds whose start and end nothing covers; fewer waves with less LDS
+// put several units on a CU, each slower (balanced / 2 / 4 / 8 waves):
+//   head_dim 128, 512 units x 64 14.6 / 6.6 / 6.4 / 10.0, x 256 21.7 / 15.6 /
+//   15.1 / 18.0, x 512 30.7 / - / 25.2 / 27.0; 1024 x 64 15.1 / 9.9 / 14.1 /
+//   22.4, x 128 20.3 / 17.0 / 18.1 / 25.7, x 512 49.6 / - / 44.7 / 49.7; 1536 x
+//   128 28.7 / 25.4 / 25.5 / 39.6, x 256 43.6 / 41.1 / 38.8 / 50.2, x 512 75.1 /
+//   - / 80.1; 2048 x 64 22.8 / 22.6 / 30.2.
+//   head_dim 64, 1024 x 64 13.7 / 6.1 / 6.6 / 10.7, x 512 31.2 / - / 26.4 / 26.3;
+//   2048 x 64 15.2 / 11.0 / 15.7, x 512 50.2 / - / 48.4. head_dim 256, 512 x 256
+//   30.3 / 24.1 / 26.2 / 26.1; 1024 x 256 53.1 / 46.4 / 50.7.
+// Lengths spread from a twentieth of the longest on favour the balanced schedule:
+//   head_dim 128, 1024 x up to 512 32.8 / - / 30.0, 1536 x up to 256 28.2 / 28.6 /
+//   30.0; head_dim 64, 2048 x up to 512 36.3 / - / 36.6; head_dim 256, 512 x up to
+//   256 23.7 / 18.9, 1024 x up to 256 35.0 / 38.3; so the line lies at 1024 eight-
+//   wave workgroups, 512 at head_dim 256.
+namespace {
+// Waves of a unit's workgroup; 0: the balanced schedule.
+int unit_waves(const gk_decode_params* p, int64_t units) {
   const int64_t visible = p->sliding_window > 0 ? std::min(p->max_context, p->sliding_window) : p->max_context;
+  const int64_t load = p->head_dim == 64 ? (units + 1) / 2 : units;  // eight-wave workgroups in CUs
+  if (load > 256) {
+    if (p->head_dim == 256) {
+      if (load <= 512 && visible <= unit_short_keys(2)) return 2;
+    } else if (load <= 512) {
+      if (visible <= unit_short_keys(4)) return 4;
+    } else if (load <= 1024) {
+      if (visible <= unit_short_keys(2) / 2) return 2;
+      if (visible <= unit_short_keys(4)) return 4;
+    }
+  }
   const int64_t most = units < 32 ? std::min(2048, (3 << 16) / p->head_dim) : unit_max_keys(p->head_dim);
-  return visible <= most && units <= 512 && units * visible * p->head_dim <= int64_t(1) << 26;
+  return visible <= most && units <= 512 && units * visible * p->head_dim <= int64_t(1) << 26 ? 8 : 0;
 }
+}  // namespace
+
+bool unit_decode_fits(const gk_decode_params* p, int64_t units) { return unit_waves(p, units) != 0; }
 
 int launch_unit_decode(const DecodeArgs& a, bool softcap, int head_dim, const gk_decode_params* p, bool store,
                        hipStream_t stream) {
@@ -383,11 +416,18 @@ int launch_unit_decode(const DecodeArgs& a, bool softcap, int head_dim, const gk
     ua.slot_mapping = p->slot_mapping;
     ua.d.pool_out = static_cast<uint16_t*>(const_cast<void*>(p->pool));
   }
-  const dim3 grid((unsigned)(a.rows * ua.units_per_row));
+  const int64_t units = (int64_t)a.rows * ua.units_per_row;
+  const dim3 grid((unsigned)units);
+  const int waves = unit_waves(p, units);
+  const auto launch_waves = [&](auto d, auto w) {
+    constexpr int D = decltype(d)::value, W = decltype(w)::value;
+    if (softcap) decode_unit_kernel<D, true, W><<<grid, W * 64, 0, stream>>>(ua);
+    else decode_unit_kernel<D, false, W><<<grid, W * 64, 0, stream>>>(ua);
+  };
   const auto launch = [&](auto d) {
-    constexpr int D = decltype(d)::value;
-    if (softcap) decode_unit_kernel<D, true><<<grid, kUnitWaves * 64, 0, stream>>>(ua);
-    else decode_unit_kernel<D, false><<<grid, kUnitWaves * 64, 0, stream>>>(ua);
+    if (waves == 2) launch_waves(d, std::integral_constant<int, 2>{});
+    else if (waves == 4) launch_waves(d, std::integral_constant<int, 4>{});
+    else launch_waves(d, std::integral_constant<int, 8>{});
   };
   if (head_dim == 64) launch(std::integral_constant<int, 64>{});
   else if (head_dim == 128) launch(std::integral_constant<int, 128>{});

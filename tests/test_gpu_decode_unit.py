@@ -118,6 +118,21 @@ def test_lengths_around_the_rule(runner, d, few, many, block, above):
     step(runner, 4, 1, d, block, [many + above, many - 33] + [5] * 30)
 
 
+@pytest.mark.parametrize("heads,kv_heads,d,rows,longest", [
+    (32, 8, 128, 33, 512), (32, 8, 128, 33, 513),      # four waves, then eight
+    (32, 8, 128, 65, 128), (32, 8, 128, 65, 129),      # two waves, then four
+    (8, 8, 128, 128, 512), (8, 8, 128, 128, 513),      # four waves, then the balanced schedule
+    (8, 8, 128, 129, 100),                             # more units than the unit form takes
+    (32, 8, 64, 65, 200), (32, 8, 64, 130, 128),
+    (16, 8, 256, 33, 256), (16, 8, 256, 33, 257), (16, 8, 256, 65, 40),
+])
+@pytest.mark.parametrize("window", [-1, 60])
+def test_many_units(runner, heads, kv_heads, d, rows, longest, window):
+    rng = np.random.default_rng(rows + longest)
+    step(runner, heads, kv_heads, d, 16, [longest, longest - 1] + list(rng.integers(0, 48, rows - 2)), window=window,
+         skip=(2,))
+
+
 def test_window_inside_a_page_at_the_limit(runner):
     # 2048 visible keys that start inside a page: one block-table entry more than keys / page.
     step(runner, 4, 1, 128, 16, [3001, 2500] + [9] * 30, window=2048)
