@@ -81,7 +81,7 @@ def _call_directly(torch):
 
     For an operator with a custom-class argument, ``torch.ops.gaudirt.op(...)``
     looks through all call arguments, as a tree, for the stand-ins that export
-    and fake tracing use: 6 us of the 18.7 us of a small attention call. These
+    and fake tracing use: 6 us of the 18.7 us that a small attention call took with it. These
     operators have exactly one such argument, the metadata; when it is the real
     object the search finds nothing and the registered operator is called next,
     which is all that happens here. Every other call (metadata by keyword, a

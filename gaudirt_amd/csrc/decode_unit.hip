@@ -5,13 +5,14 @@
 // bytes: the balanced schedule (decode_stream.hip) takes a kernel for the KV
 // store, one for the attention and one for the merge, about 4 us of stream time
 // and 3.5 us of host time each, for 8 us of work. In one launch 8 units of 64
-// keys take 4.9 us instead of 10.0, 256 units of 512 keys 14.2 instead of 20.9
+// keys take 5.0 us instead of 10.5, 256 units of 512 keys 13.9 instead of 21.0
 // (head_dim 128, with the store, on the stream); what then bounds it is the
 // chain of round trips: arguments, the row's fields, its table and query, then
-// 1.5 us for every 256 keys. Here the eight waves of a
-// workgroup share one unit (row, kv head, head group): wave w takes the unit's
-// key tiles w, w + 8, ..., and the waves' softmax states meet in LDS. Nothing is
-// split across workgroups, so there is no workspace and no merge launch.
+// 1.5 us for every 256 keys. Here the waves of a workgroup (eight; four or two
+// for short rows of many units, so that units share a CU) share one unit (row,
+// kv head, head group): wave w takes every WAVES-th of the unit's key tiles, and
+// the waves' softmax states meet in LDS. Nothing is split across workgroups, so
+// there is no workspace and no merge launch.
 //
 // The KV store of the new rows rides along: the workgroup of (row, kv head)
 // writes the row's key and value into the pool, and every workgroup takes the
@@ -23,8 +24,8 @@
 // tiles, a re-base at every new running maximum, probabilities rounded to bf16,
 // P . V from a transposed LDS read, fp32 accumulation. The K and V tiles of a
 // wave are 16-byte direct loads into one LDS stage; the next K tile is issued
-// once this one is in registers, the next V tile after P . V, and the eight
-// waves cover each other's waits.
+// once this one is in registers, the next V tile after P . V, and the waves
+// of a CU cover each other's waits.
 #include "decode_common.hpp"
 
 #include <algorithm>
