@@ -822,7 +822,8 @@ int paged_decode(const gk_decode_params* p, void* workspace, size_t workspace_by
   }
   const int32_t part = decode_partition(p);
   const int32_t max_parts = decode_max_parts(p);
-  const size_t need = unit ? 0 : decode_workspace_bytes(p);
+  // The unit kernel uses none of it; what a caller has to bring does not depend on that choice.
+  const size_t need = decode_workspace_bytes(p);
   if (need > workspace_bytes || (need && !workspace))
     return fail(GK_ERR_WORKSPACE, "gk_paged_decode: workspace too small (" + std::to_string(need) + " bytes needed)");
   const int group = p->q_heads / p->kv_heads;

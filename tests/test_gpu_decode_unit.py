@@ -153,3 +153,26 @@ def test_contexts_beyond_max_context(runner):
     torch.cuda.synchronize()
     del ws
     orc.check_tolerance(runner.bits_of(out), orc.direct_bf16_pv(case.oracle_problem()), MAX_ABS, MEAN_ABS)
+
+
+def test_short_workspace_stays_refused(runner):
+    """The workspace that the size query names has to be there although this path leaves it untouched."""
+    import ctypes
+
+    import torch
+    from gaudirt_amd import capi
+
+    case = cases.decode_case(3, 2, 8, 2, 128, 16, 16, np.array([40, 64]))
+    q, pool, tables = runner.bf16_device(case.query), runner.bf16_device(case.pool), runner.to_device(case.block_tables)
+    lens = runner.to_device(case.lens.astype(np.int32))
+    out = torch.full((2, 8 * 128), 3.0, dtype=torch.bfloat16, device="cuda")
+    params = runner.decode_params(q, pool, tables, lens, 8, 2, 128, 16, case.scale, out)
+    lib = capi.load()
+    need = lib.gk_paged_decode_workspace_bytes(ctypes.byref(params))
+    assert need > 0
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    for pointer, size in ((ws.data_ptr(), need - 1), (None, need), (None, 0)):
+        rc = lib.gk_paged_decode(ctypes.byref(params), ctypes.c_void_p(pointer), size, capi.current_stream())
+        assert rc == capi.GK_ERR_WORKSPACE, (size, rc)
+    torch.cuda.synchronize()
+    assert (out == 3.0).all()
