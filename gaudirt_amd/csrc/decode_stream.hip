@@ -764,6 +764,8 @@ __device__ __forceinline__ void decode_stream_body(StreamArgs sa) {
       for (int c = 0; c < S::NC; ++c) sc[h] = mfma32(kr[h][c], qb[c], sc[h]);
     }
 
+    if constexpr (!SOFTCAP) mfma_results_ready(sc);
+
     // Mask, and the row maximum over this lane's scores. Without softcap the
     // scores stay raw: a tile whose keys are all visible needs no per-element
     // mask, the maximum is compared with (m_run + kDecodeRescaleSlack) / scale

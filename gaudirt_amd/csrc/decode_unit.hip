@@ -227,7 +227,7 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_unit_kernel(UnitArgs ua)
 #pragma unroll
       for (int c = 0; c < S::NC; ++c) sc[g] = mfma32(kr[g][c], qb[c], sc[g]);
     }
-    mfma_results_ready(sc);
+    if constexpr (!SOFTCAP) mfma_results_ready(sc);
     const bool inside = !SOFTCAP && tb >= rt.left && tb + TS <= rt.ctx;
     if (!inside) {
 #pragma unroll

@@ -90,16 +90,34 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
   return r;
 }
 // The wait states between an MFMA and a read of its result by inline asm (max2,
-// max3): a matrix result reaches the registers several issue slots later, the
-// compiler counts them for its own instructions only, and asm that comes sooner
-// reads the value before the last accumulation. Needed where the maxima can
-// follow the MFMAs directly, with no compiler-visible instruction on the scores
-// or a dozen others between.
+// max3): the result of a 16x16 product reaches the registers 8 issue slots later
+// (what the compiler puts before a read of its own), the compiler counts them
+// for its own instructions only, and asm that comes sooner reads the value
+// before the last accumulation. Every softmax that takes its maxima from raw
+// scores passes them through here first: where the maxima end up behind the
+// products is the scheduler's choice, and whether a copy out of an accumulation
+// register lies between is the allocator's. All tiles go through one statement,
+// which none of the maxima can precede; its comment names their registers
+// (tests/test_asm_waits.py follows them through the listing). Costs nothing that
+// shows in decode and at head_dim 256, 0.3 to 0.4% of prefill at 128 (eight
+// 512-row chunks on a 2048-token prefix: 148.8 -> 149.3 us).
 template <int N>
 __device__ __forceinline__ void mfma_results_ready(f32x4_t (&x)[N]) {
   static_assert(N == 1 || N == 2, "one or two tiles");
-  if constexpr (N == 1) asm volatile("s_nop 15" : "+v"(x[0]));
-  else asm volatile("s_nop 15" : "+v"(x[0]), "+v"(x[1]));
+  if constexpr (N == 1) asm volatile("s_nop 7 ; %0" : "+v"(x[0]));
+  else asm volatile("s_nop 7 ; %0 %1" : "+v"(x[0]), "+v"(x[1]));
+}
+template <int N, int M>
+__device__ __forceinline__ void mfma_results_ready(f32x4_t (&x)[N][M]) {
+  static_assert((N == 2 && (M == 1 || M == 2)) || (N == 4 && M == 2), "two, four or eight tiles");
+  if constexpr (M == 1)
+    asm volatile("s_nop 7 ; %0 %1" : "+v"(x[0][0]), "+v"(x[1][0]));
+  else if constexpr (N == 2)
+    asm volatile("s_nop 7 ; %0 %1 %2 %3" : "+v"(x[0][0]), "+v"(x[0][1]), "+v"(x[1][0]), "+v"(x[1][1]));
+  else
+    asm volatile("s_nop 7 ; %0 %1 %2 %3 %4 %5 %6 %7"
+                 : "+v"(x[0][0]), "+v"(x[0][1]), "+v"(x[1][0]), "+v"(x[1][1]), "+v"(x[2][0]), "+v"(x[2][1]),
+                   "+v"(x[3][0]), "+v"(x[3][1]));
 }
 
 // Maximum of N >= 2 values as a tree of bare max3 (depth log3 N): a chain

@@ -452,14 +452,7 @@ __global__ __launch_bounds__(kPrefillWaves * 64, 1) void prefill_kernel(PrefillA
   // scores (scale > 0), and p = exp2(fma(s, scale, -max)).
   auto softmax = [&](int tb) __attribute__((always_inline)) {
     const bool full = tb + kKeys - 1 <= wave_pos_min && tb >= wave_left_max;
-    // At head_dim 256 the maxima can come two issue slots after the scores (at
-    // 128 the early V reads lie between, at 64 the P.V products and a barrier).
-    if constexpr (D == 256 && !SOFTCAP) {
-      f32x4_t last[2] = {sc[0][0], sc[1][0]};
-      mfma_results_ready(last);
-      sc[0][0] = last[0];
-      sc[1][0] = last[1];
-    }
+    if constexpr (!SOFTCAP) mfma_results_ready(sc);
     // Mask, and each tile's row maximum over this lane's 4 kKG scores.
     float mx[kNT];
 #pragma unroll
