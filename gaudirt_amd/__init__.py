@@ -17,10 +17,11 @@ for it (python/gaudirt/__init__.py, src/bridge/generic_private_use1.cpp:430-540)
 - ``set_batch_invariant_decode(enabled, partition_tokens=2048)``: decode rows
   of ``paged_attn`` on fixed split-K partitions, so each row's output is a
   function of that row alone, bit for bit (the reference's single-row replay,
-  tests/paged_attention_smoke.py:145-150); off by default, where the balanced
-  schedule's split points depend on the whole batch. The environment variable
-  ``GAUDIRT_AMD_BATCH_INVARIANT_DECODE`` (``1``, or a partition in keys) turns
-  it on when the extension loads.
+  tests/paged_attention_smoke.py:145-150), and prefill chunks with their keys
+  in one piece, so each chunk's output is a function of that chunk alone; off
+  by default, where the schedules' split points depend on the whole batch. The
+  environment variable ``GAUDIRT_AMD_BATCH_INVARIANT_DECODE`` (``1``, or a
+  partition in keys) turns it on when the extension loads.
 
 The extension is loaded on first use of any of these names (or by
 ``load_extension()``); a missing build raises ImportError. There is no other
@@ -66,8 +67,10 @@ def load_extension():
 
 def set_batch_invariant_decode(enabled=True, partition_tokens=BATCH_INVARIANT_PARTITION):
     """Decode rows of paged_attn on fixed partitions of `partition_tokens` keys (a
-    multiple of 32 up to 8192): every row's output then depends on that row alone.
-    Off: the library's balanced schedule (the default; faster on skewed batches)."""
+    multiple of 32 up to 8192) and prefill rows with their keys in one piece: every
+    row's output then depends on its own sequence alone. Off: the library's
+    schedules (the default; faster on skewed batches and on few prefill rows),
+    whose split points follow the whole batch."""
     load_extension()._set_decode_partition(int(partition_tokens) if enabled else 0)
 
 

@@ -31,7 +31,7 @@ STREAM_UNIT_COST = 2
 EXPORTED = [
     "gk_last_error", "gk_version", "gk_kv_store", "gk_paged_decode_workspace_bytes",
     "gk_paged_decode_partition_tokens", "gk_paged_decode", "gk_paged_decode_scratch", "gk_paged_prefill",
-    "gk_prefill_list_build", "gk_prefill_list_workspace_bytes", "gk_paged_prefill_listed",
+    "gk_prefill_list_build", "gk_prefill_list_build_uncut", "gk_prefill_list_workspace_bytes", "gk_paged_prefill_listed",
     "gk_split_k_merge",
     "gk_attn_tile_indices", "gk_advance_decode_lengths",
     "gk_metadata_workspace_bytes", "gk_metadata_normalize", "gk_block_tables",
@@ -164,7 +164,8 @@ def load():
     lib.gk_paged_decode.argtypes = [ctypes.POINTER(DecodeParams), c_void_p, ctypes.c_size_t, c_void_p]
     lib.gk_paged_decode_scratch.argtypes = [ctypes.POINTER(DecodeParams), c_void_p]
     lib.gk_paged_prefill.argtypes = [ctypes.POINTER(PrefillParams), c_void_p]
-    lib.gk_prefill_list_build.argtypes = [c_void_p] * 3 + [c_i32] * 5 + [c_void_p, c_i64, ctypes.POINTER(PrefillList)]
+    for build in (lib.gk_prefill_list_build, lib.gk_prefill_list_build_uncut):
+        build.argtypes = [c_void_p] * 3 + [c_i32] * 5 + [c_void_p, c_i64, ctypes.POINTER(PrefillList)]
     lib.gk_prefill_list_workspace_bytes.restype = ctypes.c_size_t
     lib.gk_prefill_list_workspace_bytes.argtypes = [ctypes.POINTER(PrefillParams), ctypes.POINTER(PrefillList)]
     lib.gk_paged_prefill_listed.argtypes = [ctypes.POINTER(PrefillParams), ctypes.POINTER(PrefillList), c_void_p,

@@ -986,8 +986,8 @@ int paged_prefill_listed(const gk_prefill_params* p, const gk_prefill_list* list
 }
 
 int prefill_list_build(const int32_t* seq_first_row, const int32_t* seq_rows, const int32_t* seq_prefix, int32_t seqs,
-                       int32_t q_heads, int32_t kv_heads, int32_t head_dim,
-                       int32_t sliding_window, int32_t* words, int64_t capacity, gk_prefill_list* list) {
+                       int32_t q_heads, int32_t kv_heads, int32_t head_dim, int32_t sliding_window, bool cut,
+                       int32_t* words, int64_t capacity, gk_prefill_list* list) {
   if (!list || list->struct_size != sizeof(gk_prefill_list))
     return fail(GK_ERR_INVALID_ARGUMENT, "gk_prefill_list_build: struct_size does not match this library's gk_prefill_list");
   if ((head_dim != 64 && head_dim != 128 && head_dim != 256) || q_heads <= 0 || kv_heads <= 0 || q_heads % kv_heads ||
@@ -1007,8 +1007,10 @@ int prefill_list_build(const int32_t* seq_first_row, const int32_t* seq_rows, co
     std::vector<PrefillSeq> in(seqs);
     for (int32_t s = 0; s < seqs; ++s)
       in[s] = {seq_first_row[s], seq_rows[s], seq_prefix[s]};
-    const PrefillWorkList work = prefill_work_list(in.data(), seqs, q_heads / kv_heads, kv_heads, head_dim,
-                                                   sliding_window, device_cus());
+    const int group = q_heads / kv_heads;
+    const PrefillWorkList work =
+        cut ? prefill_work_list(in.data(), seqs, group, kv_heads, head_dim, sliding_window, device_cus())
+            : prefill_whole_list(in.data(), seqs, group, head_dim, sliding_window);
     list->item_count = (int32_t)work.items.size();
     list->merge_count = (int32_t)work.merges.size();
     list->part_slots = work.slots;
@@ -1037,7 +1039,16 @@ extern "C" int gk_prefill_list_build(const int32_t* seq_first_row, const int32_t
                                      int32_t sliding_window, int32_t* words, int64_t capacity, gk_prefill_list* list) {
   gk::clear_error();
   return gk::prefill_list_build(seq_first_row, seq_rows, seq_prefix, seqs, q_heads, kv_heads, head_dim, sliding_window,
-                                words, capacity, list);
+                                true, words, capacity, list);
+}
+
+extern "C" int gk_prefill_list_build_uncut(const int32_t* seq_first_row, const int32_t* seq_rows,
+                                           const int32_t* seq_prefix, int32_t seqs, int32_t q_heads, int32_t kv_heads,
+                                           int32_t head_dim, int32_t sliding_window, int32_t* words, int64_t capacity,
+                                           gk_prefill_list* list) {
+  gk::clear_error();
+  return gk::prefill_list_build(seq_first_row, seq_rows, seq_prefix, seqs, q_heads, kv_heads, head_dim, sliding_window,
+                                false, words, capacity, list);
 }
 
 extern "C" size_t gk_prefill_list_workspace_bytes(const gk_prefill_params* params, const gk_prefill_list* list) {

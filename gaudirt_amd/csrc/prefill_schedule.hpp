@@ -109,20 +109,28 @@ inline void prefill_cut(PrefillWorkList& out, const PrefillItem& whole, const st
   }
 }
 
-inline PrefillWorkList prefill_work_list(const PrefillSeq* seqs, int count, int group, int kv_heads, int head_dim,
-                                         int window, int cus) {
+// Every row tile whole: a row's keys are taken in one order whatever else the
+// list holds, so its output depends on its own sequence alone.
+inline PrefillWorkList prefill_whole_list(const PrefillSeq* seqs, int count, int group, int head_dim, int window) {
   const int keys = prefill_step_keys(head_dim), tile_rows = prefill_tile_qrows(head_dim) / group;
   PrefillWorkList whole;
-  int64_t total = 0;
   for (int s = 0; s < count; ++s)
     for (int r0 = 0; r0 < seqs[s].rows; r0 += tile_rows) {
       const int nr = std::min(tile_rows, seqs[s].rows - r0), pos = seqs[s].prefix + r0;
       const int left = window > 0 ? std::max(0, pos - window + 1) : 0, key0 = left / keys * keys;
       const int steps = (pos + nr - key0 + keys - 1) / keys;
       whole.items.push_back({seqs[s].first_row + r0, nr, pos, key0, steps, -1, {0, 0}});
-      total += steps;
     }
   prefill_longest_first(whole.items);
+  return whole;
+}
+
+inline PrefillWorkList prefill_work_list(const PrefillSeq* seqs, int count, int group, int kv_heads, int head_dim,
+                                         int window, int cus) {
+  const int keys = prefill_step_keys(head_dim);
+  PrefillWorkList whole = prefill_whole_list(seqs, count, group, head_dim, window);
+  int64_t total = 0;
+  for (const auto& it : whole.items) total += it.steps;
   // Every kv head has the same list, and the grid gives each an equal share of
   // the GPU: balance one head's list over its share.
   const PrefillCost cost = prefill_cost(head_dim);

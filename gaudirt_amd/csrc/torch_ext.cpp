@@ -50,7 +50,8 @@ void check_gk(int rc, const char* what) {
 // fixed partition of that many keys (the partitioned kernel) makes every
 // decode row's output a function of that row alone, bit for bit: the
 // reference's single-row replay equals the batched row
-// (tests/paged_attention_smoke.py:145-150).
+// (tests/paged_attention_smoke.py:145-150). Prefill chunks then run uncut, each
+// a function of its own sequence alone.
 std::atomic<int32_t> g_decode_partition{0};
 
 hipStream_t current_stream() { return c10::hip::getCurrentHIPStream().stream(); }
@@ -235,6 +236,8 @@ struct PlanInfo {
   // metadata's own row requests.
   int64_t prefill_items = 0, prefill_merges = 0, prefill_part_slots = 0;
   int64_t prefill_items_offset = 0, prefill_merges_offset = 0;
+  // Where that list cuts items: the same work uncut, for batch-invariant calls.
+  int64_t prefill_uncut_items = 0, prefill_uncut_offset = 0;
   at::Tensor prefill_row_request;
 };
 
@@ -793,26 +796,31 @@ class PagedMetadata : public torch::CustomClassHolder {
     if (!seq_rows.empty()) {
       gk_prefill_list list{};
       list.struct_size = sizeof(list);
-      const auto build = [&] {
-        return gk_prefill_list_build(seq_first.data(), seq_rows.data(), seq_prefix.data(),
-                                     static_cast<int32_t>(seq_rows.size()),
-                                     static_cast<int32_t>(query_heads), static_cast<int32_t>(kv_heads),
-                                     static_cast<int32_t>(head_dim), static_cast<int32_t>(window), work.data(),
-                                     static_cast<int64_t>(work.size()), &list);
+      const auto build = [&](auto list_build) {
+        work.resize(4096);
+        for (;;) {
+          const int rc = list_build(seq_first.data(), seq_rows.data(), seq_prefix.data(),
+                                    static_cast<int32_t>(seq_rows.size()), static_cast<int32_t>(query_heads),
+                                    static_cast<int32_t>(kv_heads), static_cast<int32_t>(head_dim),
+                                    static_cast<int32_t>(window), work.data(), static_cast<int64_t>(work.size()), &list);
+          const int64_t need = int64_t{8} * list.item_count + int64_t{4} * list.merge_count;
+          const bool short_of = rc == GK_ERR_WORKSPACE && need > static_cast<int64_t>(work.size());
+          if (!short_of) check_gk(rc, "GaudiRT attention: prefill work list");
+          work.resize(need);
+          if (!short_of) break;
+        }
       };
-      work.resize(4096);
-      int rc = build();
-      if (rc == GK_ERR_WORKSPACE) {
-        work.resize(int64_t{8} * list.item_count + int64_t{4} * list.merge_count);
-        rc = build();
-      }
-      check_gk(rc, "GaudiRT attention: prefill work list");
-      work.resize(int64_t{8} * list.item_count + int64_t{4} * list.merge_count);
+      build(gk_prefill_list_build);
       info->prefill_items = list.item_count;
       info->prefill_merges = list.merge_count;
       info->prefill_part_slots = list.part_slots;
       info->prefill_items_offset = append(work);
       info->prefill_merges_offset = info->prefill_items_offset + int64_t{8} * list.item_count;
+      if (info->prefill_merges) {
+        build(gk_prefill_list_build_uncut);
+        info->prefill_uncut_items = list.item_count;
+        info->prefill_uncut_offset = append(work);
+      }
       info->prefill_row_request = requests_;
     }
     // Page 1: the request map itself is the block table, read in place.
@@ -1000,6 +1008,7 @@ at::Tensor paged_attn_impl(const at::Tensor& query, const at::Tensor& key, const
   }
   const int32_t* words = plan.storage.data_ptr<int32_t>();
   const int32_t sw = sliding_window > 0 ? static_cast<int32_t>(sliding_window) : -1;
+  const int32_t partition = g_decode_partition.load(std::memory_order_relaxed);  // > 0: batch-invariant
   if (plan.prefill_items) {
     gk_prefill_params f{};
     f.struct_size = sizeof(f);
@@ -1026,6 +1035,11 @@ at::Tensor paged_attn_impl(const at::Tensor& query, const at::Tensor& key, const
     list.item_count = static_cast<int32_t>(plan.prefill_items);
     list.merge_count = static_cast<int32_t>(plan.prefill_merges);
     list.part_slots = static_cast<int32_t>(plan.prefill_part_slots);
+    if (partition > 0 && plan.prefill_merges) {
+      list.items = words + plan.prefill_uncut_offset;
+      list.item_count = static_cast<int32_t>(plan.prefill_uncut_items);
+      list.merge_count = list.part_slots = 0;
+    }
     const size_t need = gk_prefill_list_workspace_bytes(&f, &list);
     at::Tensor workspace;
     if (need) workspace = at::empty({static_cast<int64_t>(need)}, query.options().dtype(at::kByte));
@@ -1053,7 +1067,7 @@ at::Tensor paged_attn_impl(const at::Tensor& query, const at::Tensor& key, const
     p.softcap = softcap_f;
     p.sliding_window = sw;
     p.max_context = static_cast<int32_t>(plan.decode_max_context);
-    p.partition_tokens = g_decode_partition.load(std::memory_order_relaxed);
+    p.partition_tokens = partition;
     p.out = output.data_ptr();
     p.out_row_stride = output.stride(0);
     if (decode_stores) {

@@ -181,12 +181,16 @@ int gk_paged_prefill(const gk_prefill_params* params, hipStream_t stream);
  * lengths on the host: items (row tile, key range) of about equal length fill
  * the GPU also when the chunk has few rows or the last round of workgroups
  * would be partly empty; an item cut along its keys leaves fp32 partials in the
- * workspace, which a second launch merges (log-sum-exp). Replaces the reference's
- * host-side work plan (src/bridge/attention_plan.cpp:199-237,262-335).
+ * workspace, which a second launch merges (log-sum-exp). Where an item is cut
+ * depends on all sequences of the list and on the GPU's CUs, and with it the last
+ * bits of its rows; gk_prefill_list_build_uncut makes a list without cuts, with
+ * which (as with gk_paged_prefill) a row's output depends on its own sequence
+ * alone, and which needs no workspace. Replaces the reference's host-side work
+ * plan (src/bridge/attention_plan.cpp:199-237,262-335).
  *
- * gk_prefill_list_build (host only) writes the list for these sequences (host
+ * gk_prefill_list_build and _uncut (host only) write the list for these sequences (host
  * arrays, as gk_prefill_params' device arrays) and window into words:
- * item_count records of 8 words, then merge_count records of 4. It sets the
+ * item_count records of 8 words, then merge_count records of 4. They set the
  * counts of `list` also when capacity is too small (GK_ERR_WORKSPACE). The
  * caller copies the words to the device and sets items and merges to the two
  * sections, and row_request to the block-table row of every query row (device).
@@ -204,6 +208,9 @@ typedef struct gk_prefill_list {
 int gk_prefill_list_build(const int32_t* seq_first_row, const int32_t* seq_rows, const int32_t* seq_prefix,
                           int32_t seqs, int32_t q_heads, int32_t kv_heads, int32_t head_dim, int32_t sliding_window,
                           int32_t* words, int64_t capacity, gk_prefill_list* list);
+int gk_prefill_list_build_uncut(const int32_t* seq_first_row, const int32_t* seq_rows, const int32_t* seq_prefix,
+                                int32_t seqs, int32_t q_heads, int32_t kv_heads, int32_t head_dim,
+                                int32_t sliding_window, int32_t* words, int64_t capacity, gk_prefill_list* list);
 size_t gk_prefill_list_workspace_bytes(const gk_prefill_params* params, const gk_prefill_list* list);
 int gk_paged_prefill_listed(const gk_prefill_params* params, const gk_prefill_list* list, void* workspace,
                             size_t workspace_bytes, hipStream_t stream);

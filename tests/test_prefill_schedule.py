@@ -23,14 +23,14 @@ def test_work_list_covers_every_step(tmp_path):
     assert run.stdout.strip() == "OK"
 
 
-def build(rows, prefix, *, heads=(32, 8, 128), window=-1, capacity=4096):
+def build(rows, prefix, *, heads=(32, 8, 128), window=-1, capacity=4096, entry="gk_prefill_list_build"):
     lib, as_i32 = capi.load(), lambda a: np.ascontiguousarray(a, dtype=np.int32)
     rows, prefix = as_i32(rows), as_i32(prefix)
     first = as_i32(np.concatenate([[0], np.cumsum(rows)[:-1]]))
     words, lst = np.zeros(max(capacity, 1), dtype=np.int32), capi.PrefillList()
     ptr = lambda a: ctypes.c_void_p(a.ctypes.data)  # noqa: E731
-    rc = lib.gk_prefill_list_build(ptr(first), ptr(rows), ptr(prefix), len(rows), *heads, window, ptr(words), capacity,
-                                   ctypes.byref(lst))
+    rc = getattr(lib, entry)(ptr(first), ptr(rows), ptr(prefix), len(rows), *heads, window, ptr(words), capacity,
+                             ctypes.byref(lst))
     return rc, words, lst
 
 
@@ -62,3 +62,18 @@ def test_list_entry_checks():
     assert launch(ctypes.c_void_p(256), size) == capi.GK_ERR_INVALID_ARGUMENT
     lst.struct_size = 8
     assert launch(ctypes.c_void_p(256), size) == capi.GK_ERR_INVALID_ARGUMENT
+
+
+def test_uncut_list_follows_each_sequence_alone():
+    # 100 rows on a 2500-key prefix, alone and beside other chunks: the same two whole items.
+    def items(rows, prefix):
+        rc, words, lst = build(rows, prefix, entry="gk_prefill_list_build_uncut")
+        assert rc == capi.GK_OK and lst.merge_count == 0 and lst.part_slots == 0
+        return words[:8 * lst.item_count].reshape(-1, 8)
+
+    alone = items([100], [2500])
+    assert (alone[:, 5] == -1).all() and alone[:, 1].sum() == 100 and len(alone) == 2
+    beside = items([100, 64, 90], [2500, 1000, 2900])
+    assert {tuple(i) for i in alone} <= {tuple(i) for i in beside}
+    assert build([100], [2500])[2].merge_count > 0
+    assert build([100], [2500], capacity=8, entry="gk_prefill_list_build_uncut")[0] == capi.GK_ERR_WORKSPACE
