@@ -236,7 +236,8 @@ struct PlanInfo {
   // metadata's own row requests.
   int64_t prefill_items = 0, prefill_merges = 0, prefill_part_slots = 0;
   int64_t prefill_items_offset = 0, prefill_merges_offset = 0;
-  // Where that list cuts items: the same work uncut, for batch-invariant calls.
+  // Where that list cuts items: the same work uncut, for batch-invariant calls
+  // and for calls that find no memory for the partials.
   int64_t prefill_uncut_items = 0, prefill_uncut_offset = 0;
   at::Tensor prefill_row_request;
 };
@@ -1035,14 +1036,23 @@ at::Tensor paged_attn_impl(const at::Tensor& query, const at::Tensor& key, const
     list.item_count = static_cast<int32_t>(plan.prefill_items);
     list.merge_count = static_cast<int32_t>(plan.prefill_merges);
     list.part_slots = static_cast<int32_t>(plan.prefill_part_slots);
-    if (partition > 0 && plan.prefill_merges) {
+    const auto take_uncut = [&] {
       list.items = words + plan.prefill_uncut_offset;
       list.item_count = static_cast<int32_t>(plan.prefill_uncut_items);
       list.merge_count = list.part_slots = 0;
-    }
-    const size_t need = gk_prefill_list_workspace_bytes(&f, &list);
+    };
+    if (partition > 0 && plan.prefill_merges) take_uncut();
+    size_t need = gk_prefill_list_workspace_bytes(&f, &list);
     at::Tensor workspace;
-    if (need) workspace = at::empty({static_cast<int64_t>(need)}, query.options().dtype(at::kByte));
+    if (need) {
+      // Partials are worth some MiB of scratch, but no call fails for them.
+      try {
+        workspace = at::empty({static_cast<int64_t>(need)}, query.options().dtype(at::kByte));
+      } catch (const c10::OutOfMemoryError&) {
+        take_uncut();
+        need = 0;
+      }
+    }
     check_gk(gk_paged_prefill_listed(&f, &list, need ? workspace.data_ptr() : nullptr, need, stream),
              "GaudiRT attention (prefill)");
   }

@@ -3,7 +3,8 @@
 The list cuts row tiles along their keys by the work of the whole batch, so a
 chunk's last bits depend on what runs beside it. In batch-invariant mode they
 must not: the chunk alone, beside other chunks and in a plan made before the
-mode was switched on gives the same bits.
+mode was switched on gives the same bits. The same uncut list serves a call that
+finds no memory for the partial results.
 """
 
 import math
@@ -82,3 +83,33 @@ def test_chunks_are_batch_invariant_in_batch_invariant_mode(heads, kv_heads, d):
     reference = orc.direct_bf16_pv(problem)
     for out in (want, cut):
         orc.check_tolerance(out.cpu().numpy().view(np.uint16), reference, 2e-2, 2e-3)
+
+
+def test_no_memory_for_the_partials():
+    import torch
+
+    import gaudirt_amd
+
+    layer = Layer(32, 8, 128)
+    batch = layer.batch([CHUNK])
+    gaudirt_amd.set_batch_invariant_decode(True)
+    want = layer.attend(batch)
+    gaudirt_amd.set_batch_invariant_decode(False)
+    cut = layer.attend(batch)
+    assert not torch.equal(cut, want)
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    # Room for the output (1 MiB), not for 22 MiB of partials, which no free block holds either.
+    limit = torch.cuda.memory_reserved() + (8 << 20)
+    torch.cuda.set_per_process_memory_fraction(limit / torch.cuda.get_device_properties(0).total_memory)
+    try:
+        held = []
+        with pytest.raises(torch.OutOfMemoryError):
+            while len(held) < 1000:
+                held.append(torch.empty(21 << 20, dtype=torch.uint8, device="cuda"))
+        got = layer.attend(batch)
+        torch.cuda.synchronize()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(got, want)
+    assert torch.equal(layer.attend(batch), cut)
