@@ -52,18 +52,29 @@ struct PrefillWorkList {
 // with every CU busy (256 workgroups, 1 to 64 steps each): a step takes 0.57 us
 // at head_dim 64 (32 keys; two workgroups of a CU take 1.13, so one CU counts
 // as one worker), 1.6-1.75 at 128 (64 keys) and 1.3 at 256 (32 keys); a
-// workgroup's start and end 5-7 us; writing a partial instead of output rows
-// 1 us more; the merge 4 us and, per 256 partials, 3-6 us.
+// workgroup's start and end 5-7 us. What a cut costs is fitted to 26000 drawn
+// batches (up to 4096 rows on up to 20000 keys, windows, softcap), each launched
+// cut and uncut: the smallest charges with which no batch that is then cut runs
+// more than 2% longer for it (head_dim 64 and 128) or 0.2% (256, where pieces of
+// different key ranges also find less of each other's K/V in the L2: steps of a
+// cut list take 1.2 times as long); of 10765 other batches cut with them 2 ran
+// longer by more than 2% (7%, 3%). With smaller charges (8, 3 and 4 a launch,
+// 0.02 a partial) 2.7% of the batches ran up to 1.23 times as long: two chunks
+// of 410 and 343 rows, 16 q / 8 kv heads, head_dim 256, 23.6 us uncut, 29.2 cut;
+// 549 rows, 32 / 8, head_dim 128, 21.4 and 25.6. Over all of them cutting makes
+// head_dim 64 1.94 times as fast, 128 1.72, 256 1.57.
 struct PrefillCost {
   double piece;     // a workgroup's start and end
+  double step;      // a step of a cut list
   double merge;     // the merge launch
   double partial;   // writing and reading one partial slot, spread over the GPU
+  double merged;    // one split item of one kv head in the merge
   int least;        // shortest piece worth cutting
 };
 inline PrefillCost prefill_cost(int head_dim) {
-  if (head_dim == 64) return {10.0, 8.0, 0.02, 8};
-  if (head_dim == 128) return {4.0, 3.0, 0.018, 4};
-  return {4.0, 4.0, 0.022, 8};
+  if (head_dim == 64) return {10.0, 1.0, 6.0, 0.04, 0.0, 8};
+  if (head_dim == 128) return {4.0, 1.0, 4.0, 0.03, 0.0, 4};
+  return {4.0, 1.2, 5.0, 0.03, 0.06, 8};
 }
 
 // Time at which `slots` workers, each taking the next piece when it falls free,
@@ -79,6 +90,14 @@ inline double prefill_makespan(const std::vector<PrefillItem>& items, int slots,
     std::push_heap(busy.begin(), busy.end(), std::greater<double>());
   }
   return last;
+}
+
+// A list's time by these costs (of an uncut list: its makespan).
+inline double prefill_list_time(const PrefillWorkList& list, int slots, int kv_heads, const PrefillCost& cost) {
+  const double busy = prefill_makespan(list.items, slots, cost.piece);
+  if (list.merges.empty()) return busy;
+  return cost.step * (busy - cost.piece) + cost.piece + cost.merge +
+         kv_heads * (cost.partial * list.slots + cost.merged * list.merges.size());
 }
 
 inline void prefill_longest_first(std::vector<PrefillItem>& items) {
@@ -142,12 +161,11 @@ inline PrefillWorkList prefill_work_list(const PrefillSeq* seqs, int count, int 
   if (uncut <= 1.04 * (even + cost.piece) + cost.merge) return whole;
 
   PrefillWorkList best;
-  double best_time = 0.97 * uncut;
+  double best_time = uncut;
   const auto consider = [&](PrefillWorkList&& list) {
     if (list.merges.empty()) return;
     prefill_longest_first(list.items);
-    const double time = prefill_makespan(list.items, slots, cost.piece) + cost.merge +
-                        cost.partial * list.slots * kv_heads;
+    const double time = prefill_list_time(list, slots, kv_heads, cost);
     if (time < best_time) {
       best_time = time;
       best = std::move(list);
