@@ -90,7 +90,15 @@ def _call_directly(torch):
     which is all that happens here. Every other call (metadata by keyword, a
     stand-in, too few arguments) takes torch's own path, as do the overloads
     (``.default``) and all calls on a torch that keeps its operators elsewhere.
+
+    Around such a call torch.compile breaks its graph. Torch's own call frames are
+    then left alone; this one is marked so too, or Dynamo would try to compile it,
+    fail on the operator and warn.
     """
+    try:
+        from torch._C._dynamo.eval_frame import _FrameAction, _FrameExecStrategy, set_code_exec_strategy
+    except ImportError:
+        return
     real = torch.ScriptObject
 
     def direct(base, position):
@@ -102,6 +110,7 @@ def _call_directly(torch):
                     return self._op(*args, **kwargs)
                 return base.__call__(self, *args, **kwargs)
 
+        set_code_exec_strategy(Direct.__call__.__code__, _FrameExecStrategy(_FrameAction.SKIP, _FrameAction.DEFAULT))
         Direct.__name__, Direct.__qualname__, Direct.__module__ = base.__name__, base.__qualname__, base.__module__
         return Direct
 
