@@ -48,6 +48,17 @@ struct PrefillWorkList {
   int32_t slots = 0;                 // partial slots of one kv head
 };
 
+// Room for the words of any list of `tiles` row tiles: each worker's boundary
+// leaves an extra piece at most, in the two ways of cutting three a worker.
+inline int64_t prefill_row_tiles(int64_t rows, int group, int head_dim) {
+  const int tile_rows = prefill_tile_qrows(head_dim) / group;
+  return (rows + tile_rows - 1) / tile_rows;
+}
+inline int64_t prefill_words_bound(int64_t tiles, int kv_heads, int cus) {
+  const int64_t slots = std::max(1, cus / kv_heads);
+  return kPrefillItemWords * (tiles + 3 * slots + 1) + kPrefillMergeWords * std::min(tiles, 3 * slots + 1);
+}
+
 // What the choice weighs, in steps of the head dimension's kernel. Measured
 // with every CU busy (256 workgroups, 1 to 64 steps each): a step takes 0.57 us
 // at head_dim 64 (32 keys; two workgroups of a CU take 1.13, so one CU counts

@@ -36,6 +36,7 @@
 #include <vector>
 
 #include "gaudirt_amd.h"
+#include "prefill_schedule.hpp"
 
 namespace gaudirt_amd {
 namespace {
@@ -797,8 +798,12 @@ class PagedMetadata : public torch::CustomClassHolder {
     if (!seq_rows.empty()) {
       gk_prefill_list list{};
       list.struct_size = sizeof(list);
+      // Room for the list at the first try on 256 CUs: building one of 3000 items takes 0.7 ms.
+      int64_t tiles = 0;
+      for (const int32_t rows : seq_rows)
+        tiles += gk::prefill_row_tiles(rows, static_cast<int>(query_heads / kv_heads), static_cast<int>(head_dim));
       const auto build = [&](auto list_build) {
-        work.resize(4096);
+        work.resize(gk::prefill_words_bound(tiles, static_cast<int>(kv_heads), 256));
         for (;;) {
           const int rc = list_build(seq_first.data(), seq_rows.data(), seq_prefix.data(),
                                     static_cast<int32_t>(seq_rows.size()), static_cast<int32_t>(query_heads),

@@ -63,6 +63,12 @@ void check(const std::vector<gk::PrefillSeq>& seqs, int group, int kv_heads, int
   // At most one extra piece per worker and item, which bounds the workspace.
   const int slots = std::max(1, 256 / kv_heads);
   expect(list.slots <= 3 * slots + 1, "more partial slots than the workers can leave", trial);
+  int64_t row_tiles = 0;
+  for (const auto& s : seqs) row_tiles += gk::prefill_row_tiles(s.rows, group, d);
+  expect((int64_t)tiles == row_tiles, "the count of row tiles is wrong", trial);
+  expect((int64_t)(gk::kPrefillItemWords * list.items.size() + gk::kPrefillMergeWords * list.merges.size()) <=
+             gk::prefill_words_bound(row_tiles, kv_heads, 256),
+         "the list needs more words than the bound", trial);
   const auto whole = gk::prefill_whole_list(seqs.data(), (int)seqs.size(), group, d, window);
   expect(whole.merges.empty() && whole.items.size() == tiles, "an uncut list is cut", trial);
   const auto cost = gk::prefill_cost(d);
