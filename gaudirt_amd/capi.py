@@ -20,6 +20,7 @@ GK_ERR_UNSUPPORTED = 2
 GK_ERR_HIP = 3
 GK_ERR_OUT_OF_MEMORY = 4
 GK_ERR_WORKSPACE = 5
+GK_DECODE_PARTITIONED, GK_DECODE_BALANCED, GK_DECODE_UNIT = 0, 1, 2  # gk_paged_decode_schedule
 GK_DECODE_SCRATCH_BYTES = 32 << 20
 GK_METADATA_INLINE_WORDS = 768
 # Fixed cost per work unit of the balanced decode schedule, in tiles
@@ -30,8 +31,10 @@ STREAM_UNIT_COST = 2
 # Every function include/gaudirt_amd.h declares.
 EXPORTED = [
     "gk_last_error", "gk_version", "gk_kv_store", "gk_paged_decode_workspace_bytes",
-    "gk_paged_decode_partition_tokens", "gk_paged_decode", "gk_paged_decode_scratch", "gk_paged_prefill",
-    "gk_prefill_list_build", "gk_prefill_list_build_uncut", "gk_prefill_list_workspace_bytes", "gk_paged_prefill_listed",
+    "gk_paged_decode_partition_tokens", "gk_paged_decode_schedule", "gk_paged_decode", "gk_paged_decode_scratch",
+    "gk_paged_prefill",
+    "gk_prefill_list_build", "gk_prefill_list_build_uncut", "gk_prefill_list_workspace_bytes",
+    "gk_paged_prefill_listed",
     "gk_split_k_merge",
     "gk_attn_tile_indices", "gk_advance_decode_lengths",
     "gk_metadata_workspace_bytes", "gk_metadata_normalize", "gk_block_tables",
@@ -161,6 +164,8 @@ def load():
     lib.gk_paged_decode_workspace_bytes.argtypes = [ctypes.POINTER(DecodeParams)]
     lib.gk_paged_decode_partition_tokens.restype = c_i32
     lib.gk_paged_decode_partition_tokens.argtypes = [ctypes.POINTER(DecodeParams)]
+    lib.gk_paged_decode_schedule.restype = c_i32
+    lib.gk_paged_decode_schedule.argtypes = [ctypes.POINTER(DecodeParams)]
     lib.gk_paged_decode.argtypes = [ctypes.POINTER(DecodeParams), c_void_p, ctypes.c_size_t, c_void_p]
     lib.gk_paged_decode_scratch.argtypes = [ctypes.POINTER(DecodeParams), c_void_p]
     lib.gk_paged_prefill.argtypes = [ctypes.POINTER(PrefillParams), c_void_p]

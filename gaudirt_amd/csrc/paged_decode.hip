@@ -762,6 +762,10 @@ int64_t stream_units(const gk_decode_params* p) {
 // which needs no workspace and no merge.
 bool use_unit(const gk_decode_params* p) { return p->partition_tokens == 0 && unit_decode_fits(p, stream_units(p)); }
 
+int32_t decode_schedule(const gk_decode_params* p) {
+  return use_unit(p) ? GK_DECODE_UNIT : use_stream(p) ? GK_DECODE_BALANCED : GK_DECODE_PARTITIONED;
+}
+
 int32_t decode_partition(const gk_decode_params* p) {
   if (p->partition_tokens > 0) return p->partition_tokens;
   if (use_stream(p)) return 0;
@@ -805,7 +809,8 @@ size_t decode_workspace_bytes(const gk_decode_params* p) {
 int paged_decode(const gk_decode_params* p, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   if (int rc = validate(p)) return rc;
   if (p->rows == 0) return GK_OK;
-  const bool unit = use_unit(p);
+  const int32_t schedule = decode_schedule(p);
+  const bool unit = schedule == GK_DECODE_UNIT;
   bool unit_store = false;
   if (p->new_key) {
     if (!p->new_value || !p->slot_mapping)
@@ -854,7 +859,7 @@ int paged_decode(const gk_decode_params* p, void* workspace, size_t workspace_by
   a.out = static_cast<uint16_t*>(p->out);
   a.out_stride = p->out_row_stride;
   if (unit) return launch_unit_decode(a, softcap, p->head_dim, p, unit_store, stream);
-  if (use_stream(p))
+  if (schedule == GK_DECODE_BALANCED)
     return launch_stream_decode(a, softcap, p->head_dim, stream_decode_wgs(p->head_dim, softcap, p->block_size), workspace,
                                 stream);
   if (need) {
@@ -984,6 +989,13 @@ extern "C" size_t gk_paged_decode_workspace_bytes(const gk_decode_params* params
 
 extern "C" int32_t gk_paged_decode_partition_tokens(const gk_decode_params* params) {
   return params && params->struct_size == sizeof(gk_decode_params) ? gk::decode_partition(params) : 0;
+}
+
+extern "C" int32_t gk_paged_decode_schedule(const gk_decode_params* params) {
+  const bool known = params && params->struct_size == sizeof(gk_decode_params) && params->rows > 0 &&
+                     params->kv_heads > 0 && params->q_heads >= params->kv_heads &&
+                     (params->head_dim == 64 || params->head_dim == 128 || params->head_dim == 256);
+  return known ? gk::decode_schedule(params) : GK_DECODE_PARTITIONED;
 }
 
 extern "C" int gk_paged_decode(const gk_decode_params* params, void* workspace, size_t workspace_bytes,

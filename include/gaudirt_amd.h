@@ -116,6 +116,13 @@ size_t gk_paged_decode_workspace_bytes(const gk_decode_params* params);
  * short contexts, one workgroup per unit applies (the latter leaves the
  * workspace untouched). */
 int32_t gk_paged_decode_partition_tokens(const gk_decode_params* params);
+/* Which form gk_paged_decode takes for these parameters (host only). */
+enum {
+  GK_DECODE_PARTITIONED = 0,   /* fixed split-K partitions */
+  GK_DECODE_BALANCED = 1,      /* balanced split of all key tiles */
+  GK_DECODE_UNIT = 2           /* one workgroup per unit */
+};
+int32_t gk_paged_decode_schedule(const gk_decode_params* params);
 int gk_paged_decode(const gk_decode_params* params, void* workspace, size_t workspace_bytes,
                     hipStream_t stream);
 

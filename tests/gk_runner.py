@@ -60,15 +60,22 @@ def paged_decode(params):
     return ws
 
 
-def run_case(case, partition=0, out=None):
-    """Run gk_paged_decode on a host DecodeCase; returns output bf16 bits [B, Hq*d]."""
+def schedule_of(params):
+    return capi.load().gk_paged_decode_schedule(ctypes.byref(params))
+
+
+def run_case(case, partition=0, out=None, max_context=None, schedule=None):
+    """Run gk_paged_decode on a host DecodeCase, on `schedule` if given; returns output bf16 bits [B, Hq*d]."""
     q = bf16_device(case.query)
     pool = bf16_device(case.pool)
     tables = to_device(case.block_tables)
     lens = to_device(case.lens.astype(np.int32))
     out = torch.full((case.batch, case.heads * case.head_dim), float("nan"), dtype=torch.bfloat16, device="cuda")
     params = decode_params(q, pool, tables, lens, case.heads, case.kv_heads, case.head_dim, case.block_size,
-                           case.scale, out, partition=partition, softcap=case.softcap, window=case.window)
+                           case.scale, out, partition=partition, softcap=case.softcap, window=case.window,
+                           max_context=max_context)
+    if schedule is not None:
+        assert schedule_of(params) == schedule, (schedule_of(params), schedule)
     ws = paged_decode(params)
     torch.cuda.synchronize()
     del ws

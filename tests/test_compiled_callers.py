@@ -22,7 +22,8 @@ def test_no_frame_of_the_operator_call_is_compiled(name):
     metadata = torch.ops.quantized.linear_prepack(
         torch.quantize_per_tensor(torch.ones(4, 4), 0.1, 0, torch.qint8), None)
     assert type(metadata) is torch.ScriptObject
-    options = {"paged_attn": (128, 0.1), "rotary_paged_attn": (128, 128, True, 0.1), "rotary_embedding": (128, 128, True)}
+    options = {"paged_attn": (128, 0.1), "rotary_paged_attn": (128, 128, True, 0.1),
+               "rotary_embedding": (128, 128, True)}
 
     def layer(x, pool, m):
         x = x + 1

@@ -44,6 +44,22 @@ def check(case, actual, fp32_softmax=False, rows=None):
     return max_abs, mean_abs
 
 
+# A bound on every row that no form for short contexts takes.
+LONG = 1 << 17
+
+
+def run(runner, case, **kwargs):
+    """The case's output bits on the balanced schedule; where the library would take the form for short contexts
+    (tests/test_gpu_decode_unit.py), that one has to agree."""
+    from gaudirt_amd import capi
+
+    balanced = runner.run_case(case, max_context=LONG, schedule=capi.GK_DECODE_BALANCED, **kwargs)
+    chosen = runner.run_case(case, **kwargs)
+    max_abs, _ = orc.tolerance_errors(chosen, balanced)
+    assert max_abs <= 2 * MAX_ABS, max_abs
+    return balanced
+
+
 def test_library_choice_is_the_balanced_schedule(runner):
     import ctypes
     import torch
@@ -72,14 +88,14 @@ def test_stream_geometries(runner, geometry):
     block = 16 if d == 256 else 32
     case = cases.decode_case(11, len(lens), heads, kv_heads, d, block, 4096 // block * 4, lens)
     print("geometry", geometry, flush=True)
-    check(case, runner.run_case(case))
+    check(case, run(runner, case))
 
 
 @pytest.mark.parametrize("block_size", [32, 64, 256, 1024])
 def test_stream_block_sizes(runner, block_size):
     lens = np.array([5, 300, 777, 1024, 63, 2048, 1])
     case = cases.decode_case(block_size + 3, len(lens), 32, 8, 128, block_size, 8192 // block_size * 2, lens)
-    check(case, runner.run_case(case))
+    check(case, run(runner, case))
 
 
 @pytest.mark.parametrize("geometry", [(128, 1), (128, 2), (128, 4), (128, 8), (128, 16), (64, 1), (64, 4),
@@ -93,7 +109,7 @@ def test_stream_small_blocks(runner, geometry):
     lens = np.array([1, 2, 3, 4, 5, 31, 33, 300, 777, 1024, 2047])
     case = cases.decode_case(7 * block + d, len(lens), heads, kv_heads, d, block, 8192 // block * 2, lens)
     print("head_dim", d, "block", block, flush=True)
-    check(case, runner.run_case(case))
+    check(case, run(runner, case))
 
 
 @pytest.mark.parametrize("block", [1, 2, 4, 16])
@@ -144,7 +160,7 @@ def test_one_long_row_split_over_the_grid(runner):
     # 2 kv heads x 20000 keys: ~1250 tiles over ~1000 workgroups, so each unit's
     # partial states come from hundreds of workgroups.
     case = cases.decode_case(21, 1, 16, 2, 128, 128, 200, [20000])
-    check(case, runner.run_case(case))
+    check(case, run(runner, case))
 
 
 def test_many_rows_skewed(runner):
@@ -154,7 +170,7 @@ def test_many_rows_skewed(runner):
     lens = np.concatenate([rng.integers(1, 40, 150), rng.integers(1, 1300, 150), [1, 1, 2]]).astype(np.int32)
     rng.shuffle(lens)
     case = cases.decode_case(22, len(lens), 8, 2, 64, 32, 8192, lens)
-    check(case, runner.run_case(case))
+    check(case, run(runner, case))
 
 
 def test_rows_beyond_the_prefetched_windows(runner):
@@ -163,12 +179,12 @@ def test_rows_beyond_the_prefetched_windows(runner):
     rng = np.random.default_rng(17)
     lens = rng.integers(1, 400, 700).astype(np.int32)
     case = cases.decode_case(24, len(lens), 8, 2, 64, 16, int(((lens + 15) // 16).sum()) + 8, lens)
-    check(case, runner.run_case(case))
+    check(case, run(runner, case))
 
 
 def test_tiny_batch_fewer_tiles_than_workgroups(runner):
     case = cases.decode_case(23, 2, 8, 2, 128, 64, 8, [3, 40])
-    check(case, runner.run_case(case))
+    check(case, run(runner, case))
 
 
 @pytest.mark.parametrize("block", [1, 4, 32])
@@ -217,7 +233,7 @@ def test_stream_poisoned_unused_slots(runner):
         for t in range(n):
             used[case.block_tables[b, t // 32] * 32 + t % 32] = True
     case.pool[:, :, ~used, :] = 0x7fc0
-    check(case, runner.run_case(case))
+    check(case, run(runner, case))
 
 
 def test_stream_row_requests_shared(runner):
@@ -250,7 +266,7 @@ def test_stream_empty_rows_write_zeros(runner):
     lens = np.array([0, 700, 0, 33], dtype=np.int32)
     case = cases.decode_case(51, len(lens), 16, 4, 128, 32, 64, np.maximum(lens, 1))
     case.lens = lens
-    actual = runner.run_case(case)
+    actual = run(runner, case)
     assert (orc.bf16_to_f32(actual[[0, 2]]) == 0).all()
     case.lens = np.maximum(lens, 1)
     check(case, actual, rows=[1, 3])
@@ -261,7 +277,7 @@ def test_stream_matches_partitioned_path(runner):
     # tolerance, and with each other to a bf16 ulp or two).
     lens = np.array([1, 100, 4000, 2222, 31, 512])
     case = cases.decode_case(61, len(lens), 32, 8, 128, 128, 256, lens)
-    a = runner.run_case(case)
+    a = run(runner, case)
     b = runner.run_case(case, partition=512)
     check(case, a)
     check(case, b)
@@ -399,3 +415,53 @@ def test_stream_contexts_beyond_max_context_give_nan_not_stale_output(runner):
                                    capi.current_stream()))
     torch.cuda.synchronize()
     assert torch.isnan(out.float()).all()
+
+
+@pytest.mark.parametrize("heads,kv_heads,d,window", [(32, 8, 128, 2500), (16, 8, 128, 2500), (8, 8, 128, 2500),
+                                                     (14, 2, 64, 4099), (16, 8, 256, 1500)])
+@pytest.mark.parametrize("block", [1, 16, 128])
+@pytest.mark.parametrize("softcap", [0.0, 30.0])
+def test_stream_wide_windows(runner, heads, kv_heads, d, window, block, softcap):
+    # Windows wider than any that the form for short contexts takes, starting
+    # inside a tile and a page, beside rows shorter than the window and one tile.
+    from gaudirt_amd import capi
+
+    lens = np.array([6001, 5003, window + 1, window, window - 1, 40, 1, 3333])
+    case = cases.decode_case(heads + block, len(lens), heads, kv_heads, d, block, 40960 // block, lens)
+    case.window, case.softcap = window, softcap
+    print("geometry", heads, kv_heads, d, "block", block, "softcap", softcap, flush=True)
+    check(case, runner.run_case(case, schedule=capi.GK_DECODE_BALANCED), fp32_softmax=True)
+
+
+@pytest.mark.parametrize("heads,kv_heads,d", [(16, 4, 128), (2, 2, 128), (8, 2, 64), (8, 2, 256)])
+@pytest.mark.parametrize("softcap", [0.0, 30.0])
+def test_stream_narrow_windows_of_many_units(runner, heads, kv_heads, d, softcap):
+    # More units than the form for short contexts takes, of rows that see 77
+    # keys: every slot outside them is NaN.
+    import torch
+
+    from gaudirt_amd import capi
+
+    rng = np.random.default_rng(d + heads)
+    rows = {64: 2049, 128: 1025, 256: 513}[d] // kv_heads + 1
+    lens = rng.integers(1, 400, rows).astype(np.int32)
+    lens[:4] = [1, 77, 78, 399]
+    case = cases.decode_case(d, rows, heads, kv_heads, d, 16, int(((lens + 15) // 16).sum()) + 1, lens)
+    case.window, case.softcap = 77, softcap
+    used = np.zeros(case.slots, dtype=bool)
+    for b, n in enumerate(case.lens):
+        t = np.arange(max(0, int(n) - case.window), n)
+        used[case.block_tables[b, t // 16] * 16 + t % 16] = True
+    case.pool[:, :, ~used, :] = 0x7fc0
+    torch.cuda.synchronize()
+    check(case, runner.run_case(case, schedule=capi.GK_DECODE_BALANCED), fp32_softmax=True)
+
+
+def test_balanced_schedule_gives_the_same_bits_again(runner):
+    # A fully visible tile's maxima come straight after its products: a read
+    # too early would show as run-to-run differences.
+    for heads, kv_heads, d in ((32, 8, 128), (14, 2, 64), (16, 8, 256)):
+        case = cases.decode_case(d, 4, heads, kv_heads, d, 128, 200, [5000, 4999, 1, 3200])
+        first = runner.run_case(case, max_context=LONG)
+        for _ in range(5):
+            assert np.array_equal(runner.run_case(case, max_context=LONG), first), (heads, kv_heads, d)

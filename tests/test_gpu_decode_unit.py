@@ -29,9 +29,13 @@ def runner():
     return gk_runner
 
 
-def step(runner, heads, kv_heads, d, block, lens, requests=None, softcap=0.0, window=-1, skip=(), seed=0):
-    """One decode step: row r attends lens[r] keys of requests[r], its own new key last."""
+def step(runner, heads, kv_heads, d, block, lens, requests=None, softcap=0.0, window=-1, skip=(), seed=0,
+         max_context=None, unit=True):
+    """One decode step: row r attends lens[r] keys of requests[r], its own new key last. `unit`: one workgroup per
+    unit has to be what the library takes, or must not be."""
     import torch
+
+    from gaudirt_amd import capi
 
     rng = np.random.default_rng(seed + d + block + len(lens))
     lens = np.asarray(lens, dtype=np.int32)
@@ -56,7 +60,9 @@ def step(runner, heads, kv_heads, d, block, lens, requests=None, softcap=0.0, wi
     k, v = runner.bf16_device(new_k), runner.bf16_device(new_v)
     out = torch.full((rows, heads * d), float("nan"), dtype=torch.bfloat16, device="cuda")
     params = runner.decode_params(q, pool, tables, d_lens, heads, kv_heads, d, block, case.scale, out, row_request=reqs,
-                                  softcap=softcap, window=window, new_key=k, new_value=v, slot_mapping=sm)
+                                  softcap=softcap, window=window, new_key=k, new_value=v, slot_mapping=sm,
+                                  max_context=max_context)
+    assert (runner.schedule_of(params) == capi.GK_DECODE_UNIT) == unit
     ws = runner.paged_decode(params)
     torch.cuda.synchronize()
     del ws
@@ -114,8 +120,8 @@ def test_row_counts(runner, rows):
 @pytest.mark.parametrize("above", [0, 1])
 def test_lengths_around_the_rule(runner, d, few, many, block, above):
     # Fewer than 32 units and 32: each longest row on both sides of its limit.
-    step(runner, 4, 1, d, block, [few + above, few - 33, 7])
-    step(runner, 4, 1, d, block, [many + above, many - 33] + [5] * 30)
+    step(runner, 4, 1, d, block, [few + above, few - 33, 7], unit=not above)
+    step(runner, 4, 1, d, block, [many + above, many - 33] + [5] * 30, unit=not above)
 
 
 @pytest.mark.parametrize("heads,kv_heads,d,rows,longest", [
@@ -129,8 +135,9 @@ def test_lengths_around_the_rule(runner, d, few, many, block, above):
 @pytest.mark.parametrize("window", [-1, 60])
 def test_many_units(runner, heads, kv_heads, d, rows, longest, window):
     rng = np.random.default_rng(rows + longest)
+    unit = rows * kv_heads <= {64: 2048, 128: 1024, 256: 512}[d] and (longest, rows, window) != (513, 128, -1)
     step(runner, heads, kv_heads, d, 16, [longest, longest - 1] + list(rng.integers(0, 48, rows - 2)), window=window,
-         skip=(2,))
+         skip=(2,), unit=unit)
 
 
 def test_window_inside_a_page_at_the_limit(runner):
@@ -153,6 +160,24 @@ def test_contexts_beyond_max_context(runner):
     torch.cuda.synchronize()
     del ws
     orc.check_tolerance(runner.bits_of(out), orc.direct_bf16_pv(case.oracle_problem()), MAX_ABS, MEAN_ABS)
+
+
+@pytest.mark.parametrize("heads,kv_heads,rows,longest,max_context", [
+    (4, 1, 5, 2800, 100),      # eight waves: 2049 entries in LDS
+    (32, 8, 34, 700, 300),     # four: 513
+    (32, 8, 65, 300, 100),     # two: 257
+])
+@pytest.mark.parametrize("softcap", [0.0, 30.0])
+@pytest.mark.parametrize("windowed", [False, True])
+def test_steps_beyond_max_context(runner, heads, kv_heads, rows, longest, max_context, softcap, windowed):
+    # The replayed step with its store: the entries that are read in place also
+    # decide which keys are the new rows', whose slots hold NaN, and rows of one
+    # request attend each other's. With a window that still needs more entries
+    # than LDS holds.
+    lens = [longest, longest - 1, longest - 2, 100, 7] + [1 + 3 * i % max_context for i in range(rows - 5)]
+    requests = [0, 0, 0, 1, 2] + list(range(3, rows - 2))
+    step(runner, heads, kv_heads, 128, 1, lens, requests=requests, softcap=softcap, skip=(4,), max_context=max_context,
+         window=longest - 40 if windowed else -1)
 
 
 def test_short_workspace_stays_refused(runner):
