@@ -381,6 +381,21 @@ __global__ __launch_bounds__(WAVES * 64, 1) void decode_unit_kernel(UnitArgs ua)
 //   30.0; head_dim 64, 2048 x up to 512 36.3 / - / 36.6; head_dim 256, 512 x up to
 //   256 23.7 / 18.9, 1024 x up to 256 35.0 / 38.3; so the line lies at 1024 eight-
 //   wave workgroups, 512 at head_dim 256.
+// The rule sees the longest row only. Eight waves on spread lengths (balanced /
+// unit; uniform and log-uniform from a twentieth of the longest, one long row
+// among rows of a twentieth):
+//   head_dim 128, 32 units x up to 2048 14.1 / 16.5, 14.3 / 16.7, 13.5 / 16.5,
+//   x up to 1024 12.4 / 10.8, 12.0 / 10.8, 11.9 / 10.9; 128 x up to 2048 25.1 /
+//   20.9, 18.2 / 18.0, 13.9 / 17.3; 256 x up to 2048 32.4 / 26.3, 25.9 / 22.4,
+//   17.4 / 18.7. head_dim 64, 32 x up to 3072 13.6 / 15.8, 13.0 / 15.7, 12.1 /
+//   15.8; 256 x up to 3072 26.6 / 22.6, 23.7 / 20.8, 17.2 / 18.4. head_dim 256,
+//   32 x up to 1024 14.4 / 16.9, 13.6 / 16.7, 14.6 / 17.2; 256 x up to 1024
+//   37.2 / 29.9, 27.6 / 23.7, 15.7 / 18.1.
+// So a few long rows among short ones lose up to 3.7 us of stream time here, more
+// than equal lengths do, and the whole operator call still gains: 4 rows of which
+// one has 2048 keys 16.6 us instead of 21.9 for the three launches, one of 16
+// 17.2 instead of 22.3. A caller whose stream alone counts (replayed graphs) gets
+// the balanced schedule with a max_context above the limit.
 namespace {
 // Waves of a unit's workgroup; 0: the balanced schedule.
 int unit_waves(const gk_decode_params* p, int64_t units) {
