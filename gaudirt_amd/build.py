@@ -34,7 +34,7 @@ COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-I", str(ROOT
           "-Wall", "-Wno-unused-function", *DEFINES]
 
 LIB_SOURCES = ["gk_api.cpp", "block_allocator_core.cpp", "block_allocator.cpp", "kv_store.hip", "paged_decode.hip", "decode_stream.hip",
-               "decode_unit.hip",               "paged_prefill.hip", "metadata.hip", "rotary.hip"]
+               "decode_unit.hip", "paged_prefill.hip", "metadata.hip", "rotary.hip"]
 LIB_NAME = "libgaudirt_amd.so"
 
 

@@ -34,7 +34,10 @@ class Layer:
         self.pool = gaudirt_amd.allocate_paged_kv(1, self.slots, kv_heads, d)
         self.pool.normal_(generator=gen)
         self.pools = gaudirt_amd.kv_pool_views(self.pool, 0)
-        draw = lambda n: torch.randn(4, self.context, n * d, generator=gen, device="cuda").to(torch.bfloat16)  # noqa: E731
+
+        def draw(n):
+            return torch.randn(4, self.context, n * d, generator=gen, device="cuda").to(torch.bfloat16)
+
         self.q, self.k, self.v = draw(heads), draw(kv_heads), draw(kv_heads)
 
     def batch(self, chunks):
@@ -62,7 +65,8 @@ def test_chunks_are_batch_invariant_in_batch_invariant_mode(heads, kv_heads, d):
     from tests.test_prefill_schedule import build
 
     for chunks in ([CHUNK], [CHUNK, *OTHERS]):
-        _, _, lst = build([n for _, _, n in chunks], [p for _, p, _ in chunks], heads=(heads, kv_heads, d), capacity=1 << 16)
+        _, _, lst = build([n for _, _, n in chunks], [p for _, p, _ in chunks], heads=(heads, kv_heads, d),
+                          capacity=1 << 16)
         assert lst.merge_count, "the list of these chunks is to be cut"
     layer = Layer(heads, kv_heads, d)
     alone, beside = layer.batch([CHUNK]), layer.batch([CHUNK, *OTHERS])
